@@ -37,6 +37,11 @@ struct NormArgs {
 };
 
 hipError_t launch_rms_norm_f32(hipStream_t stream, NormMode mode, Reduction red, const NormArgs& a);
+// Row-per-workgroup engines (norm_row_kernels.hip) for 16-byte aligned
+// operands and hidden % 4 == 0: whether they are the ones for this shape, and
+// their launch.
+bool rms_row_engine(const NormArgs& a, bool tree);
+hipError_t launch_rms_norm_row_f32(hipStream_t stream, NormMode mode, bool tree, const NormArgs& a);
 hipError_t launch_rms_norm_groups_stable_f32(hipStream_t stream, Reduction red, float* values,
                                              const float* weight, uint32_t width, uint32_t groups,
                                              float epsilon);

@@ -26,7 +26,7 @@
 //    (kernels.metal:119-133).  Tolerance-level against the CPU operator.
 #include "device_common.hpp"
 #include "launch.hpp"
-
+#include "norm_params.hpp"
 
 namespace atlas {
 namespace {
@@ -56,26 +56,6 @@ __device__ __forceinline__ float epilogue(const NormArgs& a, size_t idx, float x
     // kNormAddScale: out aliases state
     return (a.out[idx] + n) * scale;
 }
-
-// Kernel parameters of the NormArgs engines.  A by-value struct is not
-// preloaded into SGPRs, so the fields are passed one by one, in this order:
-// the counts and the pointers the first loads need (and epsilon) fill the
-// first 56 bytes, which arrive in user SGPRs at wave launch (kernarg
-// preload), so a wavefront's first row load waits on no scalar load; the
-// outputs written only at the end follow.  wpb (wavefronts per workgroup)
-// and pair_stride (the row distance of a wavefront's second row) come from
-// the host instead of blockDim / gridDim, which are kernarg loads too.
-#define ATLAS_NORM_KPARAMS                                                                               \
-    uint32_t p_rows, uint32_t p_hidden, uint32_t wpb, uint32_t pair_stride, const float* p_x,              \
-        const float* p_residual, const float* p_weight, float* p_out, float p_epsilon, float* p_normalized, \
-        float* p_residual_out, const float* p_scale
-#define ATLAS_NORM_UNPACK                                                                                  \
-    const NormArgs a {                                                                                     \
-        p_x, p_weight, p_residual, p_normalized, p_residual_out, p_out, p_scale, p_rows, p_hidden, p_epsilon \
-    }
-#define ATLAS_NORM_KARGS(a, wpb, pair_stride)                                                                   \
-    (a).rows, (a).hidden, (wpb), (pair_stride), (a).x, (a).residual, (a).weight, (a).out, (a).epsilon,          \
-        (a).normalized, (a).residual_out, (a).scale
 
 template <int ROWS, int MODE, bool VEC>
 __global__ __launch_bounds__(64) void rms_seq_kernel(ATLAS_NORM_KPARAMS) {
@@ -675,9 +655,10 @@ __global__ __launch_bounds__(RUN ? 64 * (kRunHelpers + 1) : 64) void rms_reg_ker
 // Register-engine configuration: rows per wavefront and the fold of the
 // chunks after the first (exact wave-parallel, or in order from LDS).  Same
 // bits either way.  Measured on MI355X:
-//  * rows < 2048 (decode batches): one row per wavefront and the parallel
-//    fold -- the in-order chain is fully exposed there (C5 decode step at
-//    256 rows: 35.9 -> 30.3 us per layer);
+//  * rows < 2048 (decode batches; the row-per-workgroup engine takes over
+//    from 257 or 513 rows, rms_row_engine): one row per wavefront and the
+//    parallel fold -- the in-order chain is fully exposed there (C5 decode
+//    step at 256 rows: 35.9 -> 30.3 us per layer);
 //  * rows >= 2048, plain RMSNorm: one row per wavefront, parallel fold
 //    ([4096, 1536]: 11.7 -> 10.6 us);
 //  * rows >= 2048 with an epilogue operand (residual, add-norm, add-scale):
@@ -809,9 +790,10 @@ hipError_t launch_tree(hipStream_t s, const NormArgs& a) {
     }
 }
 
-// Rows per wavefront for the sequential LDS engine: enough wavefronts to
-// keep every SIMD streaming (>= 2048 for large row counts), bounded by 64 KB
-// of LDS.
+// Rows per wavefront for the sequential LDS engine on rows of any alignment:
+// enough wavefronts to keep every SIMD streaming (>= 2048 for large row
+// counts), bounded by 64 KB of LDS.  Aligned rows come here only past the
+// row-per-workgroup engine's width, one per wavefront.
 int pick_rows(uint32_t rows, uint32_t hidden) {
     int best = 1;
     for (int r : {2, 4, 8, 16}) {
@@ -822,28 +804,24 @@ int pick_rows(uint32_t rows, uint32_t hidden) {
     return best;
 }
 
-template <int ROWS, int MODE>
-hipError_t launch_seq_rows(hipStream_t s, const NormArgs& a, bool vec) {
-    const uint32_t stride = vec ? a.hidden + 4 : a.hidden + 1;
+template <int ROWS, int MODE, bool VEC>
+hipError_t launch_seq_rows(hipStream_t s, const NormArgs& a) {
+    const uint32_t stride = VEC ? a.hidden + 4 : a.hidden + 1;
     const size_t lds = (static_cast<size_t>(ROWS) * stride + ROWS) * sizeof(float);
     const dim3 grid((a.rows + ROWS - 1) / ROWS);
-    if (vec)
-        hipLaunchKernelGGL((rms_seq_kernel<ROWS, MODE, true>), grid, dim3(kWave), lds, s,
-                           ATLAS_NORM_KARGS(a, 1u, 0u));
-    else
-        hipLaunchKernelGGL((rms_seq_kernel<ROWS, MODE, false>), grid, dim3(kWave), lds, s,
-                           ATLAS_NORM_KARGS(a, 1u, 0u));
+    hipLaunchKernelGGL((rms_seq_kernel<ROWS, MODE, VEC>), grid, dim3(kWave), lds, s, ATLAS_NORM_KARGS(a, 1u, 0u));
     return hipGetLastError();
 }
 
 template <int MODE>
 hipError_t launch_seq(hipStream_t s, const NormArgs& a, bool vec) {
+    if (vec) return launch_seq_rows<1, MODE, true>(s, a);
     switch (pick_rows(a.rows, a.hidden)) {
-        case 16: return launch_seq_rows<16, MODE>(s, a, vec);
-        case 8: return launch_seq_rows<8, MODE>(s, a, vec);
-        case 4: return launch_seq_rows<4, MODE>(s, a, vec);
-        case 2: return launch_seq_rows<2, MODE>(s, a, vec);
-        default: return launch_seq_rows<1, MODE>(s, a, vec);
+        case 16: return launch_seq_rows<16, MODE, false>(s, a);
+        case 8: return launch_seq_rows<8, MODE, false>(s, a);
+        case 4: return launch_seq_rows<4, MODE, false>(s, a);
+        case 2: return launch_seq_rows<2, MODE, false>(s, a);
+        default: return launch_seq_rows<1, MODE, false>(s, a);
     }
 }
 
@@ -1316,7 +1294,8 @@ hipError_t launch_f16_vec(hipStream_t s, bool tree, const uint16_t* x, const uin
 }  // namespace
 
 // Engine choice.  kSequential: the sequential fold everywhere (register
-// engine, or the LDS engine for hidden > 2048 or unaligned rows).  kAuto
+// engine, the row-per-workgroup engine where rms_row_engine says so, or the
+// LDS engine for hidden > 8192 or unaligned rows).  kAuto
 // (the default): the tree engine where the output is a plain scaled row
 // (RMSNorm, the add-norm's y), the sequential fold where an epilogue
 // cancels (residual add, PLE add-scale), whose elementwise error would
@@ -1328,6 +1307,7 @@ hipError_t launch_rms_norm_f32(hipStream_t stream, NormMode mode, Reduction red,
                      (!a.residual_out || aligned16(a.residual_out));
     const bool cancels = mode == kNormResidual || mode == kNormAddScale;
     const bool tree = red == kWide || (red == kAuto && !cancels);
+    if (vec && rms_row_engine(a, tree)) return launch_rms_norm_row_f32(stream, mode, tree, a);
     if (tree && vec && a.hidden <= 2048) {
         switch (mode) {
             case kNormPlain: return launch_tree<kNormPlain>(stream, a);
