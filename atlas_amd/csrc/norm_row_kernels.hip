@@ -173,7 +173,7 @@ __global__ __launch_bounds__(64 * NW) void rms_row_exact_kernel(ATLAS_NORM_KPARA
         const float mine = lane < kBlocks ? block_sum[lane] : 0.0f;
         const float before = wave_sum_any_order_f32(lane < first ? mine : 0.0f);
         const float after = wave_sum_any_order_f32(lane < first + kRunBlocks ? mine : 0.0f);
-        // the in-order sum of <= 8704 squares is within 8704 * 2^-24 < 0.06 %
+        // the in-order sum of <= 8192 squares is within 8192 * 2^-24 < 0.05 %
         // of the estimate, so these bound its exponent from both sides
         e0 = __float_as_uint(before * 0.999f) >> 23;
         const uint32_t e1 = __float_as_uint(after * 1.001f) >> 23;

@@ -10,15 +10,11 @@
 //   NeuralOps::rope (interleaved) = rope_f32; CPU oracle cpu_rope
 //   crates/atlas-ops/tests/phase_02_operators.rs:262-272
 //
-// QK-norm+RoPE mapping on CDNA: a "unit" is one (token, head) row of
-// head_dim floats; Q heads come first, then the optional single K head.  One
-// wavefront owns UNITS consecutive units.  With head_dim = 64*V every lane
-// holds V consecutive floats of each unit in registers (one 128-bit load for
-// V = 4), and the RoPE partner x[p + d/2] of the value x[p] held by lane l
-// sits in lane l^32, so the pair is exchanged with one cross-lane swap and
-// never round-trips through memory.  The squares go to LDS for the
-// sequential fold (lane u folds unit u in index order), which makes the
-// result bit-identical to the CPU composition rms_norm -> rope.
+// QK-norm+RoPE: a "unit" is one (token, head) row of head_dim floats; Q heads
+// come first, then the optional single K head.  Wavefronts take units of one
+// token (qk_norm_rope_token_kernel, head_dim 64, 128, 256 and 512); any other
+// even head_dim, and operands off their vector's alignment, take one wavefront
+// per unit with the row in LDS.
 #include "device_common.hpp"
 #include "launch.hpp"
 
@@ -26,173 +22,31 @@
 namespace atlas {
 namespace {
 
-template <int V>
-struct vecf {
-    float v[V];
-};
-
-template <int V>
-__device__ __forceinline__ vecf<V> ldv(const float* p) {
-    vecf<V> r;
-    if constexpr (V == 2) {
-        float2 a = *reinterpret_cast<const float2*>(p);
-        r.v[0] = a.x;
-        r.v[1] = a.y;
-    } else if constexpr (V == 4) {
-        float4 a = *reinterpret_cast<const float4*>(p);
-        r.v[0] = a.x;
-        r.v[1] = a.y;
-        r.v[2] = a.z;
-        r.v[3] = a.w;
-    } else {
-#pragma unroll
-        for (int j = 0; j < V; j += 4) {
-            float4 a = *reinterpret_cast<const float4*>(p + j);
-            r.v[j] = a.x;
-            r.v[j + 1] = a.y;
-            r.v[j + 2] = a.z;
-            r.v[j + 3] = a.w;
-        }
-    }
-    return r;
-}
-
-template <int V>
-__device__ __forceinline__ void stv(float* p, const vecf<V>& r) {
-    if constexpr (V == 2) {
-        *reinterpret_cast<float2*>(p) = make_float2(r.v[0], r.v[1]);
-    } else {
-#pragma unroll
-        for (int j = 0; j < V; j += 4)
-            *reinterpret_cast<float4*>(p + j) = make_float4(r.v[j], r.v[j + 1], r.v[j + 2], r.v[j + 3]);
-    }
-}
-
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, kWave);
     return v;
 }
 
-template <int V, int UNITS, bool SEQ>
-__global__ __launch_bounds__(64) void qk_norm_rope_kernel(
-    const float* q, const float* k, const float* q_weight, const float* k_weight,
-    const float* cosine, const float* sine, float* q_out, float* k_out, uint32_t tokens,
-    uint32_t q_heads, uint32_t has_key, uint32_t rope_stride, float epsilon) {
-    constexpr uint32_t D = 64 * V;
-    constexpr uint32_t HALF = D / 2;
-    constexpr uint32_t STRIDE = D + 4;
-    __shared__ float sq[SEQ ? UNITS * STRIDE : 1];
-    __shared__ float inv_lds[UNITS];
-
-    const uint32_t lane = threadIdx.x;
-    const uint32_t total = q_heads + has_key;
-    const uint32_t units = tokens * total;
-    const uint32_t u0 = blockIdx.x * UNITS;
-    const bool low = lane < 32;
-    const uint32_t col = lane * V;                        // this lane's first column
-    const uint32_t pair = low ? col : col - HALF;         // first RoPE pair index
-    const uint32_t partner_col = low ? col + HALF : col - HALF;
-
-    vecf<V> x[UNITS];
-#pragma unroll
-    for (int u = 0; u < UNITS; ++u) {
-        const uint32_t unit = u0 + u;
-        if (unit < units) {
-            const uint32_t t = unit / total, local = unit % total;
-            const float* src = local >= q_heads ? k + static_cast<size_t>(t) * D
-                                                : q + (static_cast<size_t>(t) * q_heads + local) * D;
-            x[u] = ldv<V>(src + col);
-        } else {
-#pragma unroll
-            for (int j = 0; j < V; ++j) x[u].v[j] = 0.0f;
-        }
-    }
-
-    if constexpr (SEQ) {
-#pragma unroll
-        for (int u = 0; u < UNITS; ++u) {
-            vecf<V> s2;
-#pragma unroll
-            for (int j = 0; j < V; ++j) s2.v[j] = x[u].v[j] * x[u].v[j];
-            stv<V>(sq + u * STRIDE + col, s2);
-        }
-        __syncthreads();
-        if (lane < UNITS) {
-            const float* row = sq + lane * STRIDE;
-            float s = 0.0f;
-#pragma unroll 8
-            for (uint32_t c = 0; c < D; c += 4) {
-                float4 v = *reinterpret_cast<const float4*>(row + c);
-                s = s + v.x;
-                s = s + v.y;
-                s = s + v.z;
-                s = s + v.w;
-            }
-            inv_lds[lane] = inverse_rms(s, static_cast<float>(D), epsilon);
-        }
-        __syncthreads();
-    } else {
-#pragma unroll
-        for (int u = 0; u < UNITS; ++u) {
-            float partial = 0.0f;
-#pragma unroll
-            for (int j = 0; j < V; ++j) partial = partial + x[u].v[j] * x[u].v[j];
-            float s = wave_sum(partial);
-            if (lane == 0) inv_lds[u] = inverse_rms(s, static_cast<float>(D), epsilon);
-        }
-        __syncthreads();
-    }
-
-    const vecf<V> qw_own = ldv<V>(q_weight + col), qw_par = ldv<V>(q_weight + partner_col);
-    vecf<V> kw_own = qw_own, kw_par = qw_par;
-    if (has_key) {
-        kw_own = ldv<V>(k_weight + col);
-        kw_par = ldv<V>(k_weight + partner_col);
-    }
-
-#pragma unroll
-    for (int u = 0; u < UNITS; ++u) {
-        const uint32_t unit = u0 + u;
-        // exchange halves: lane l <-> lane l^32 (executed by the whole wave)
-        vecf<V> other;
-#pragma unroll
-        for (int j = 0; j < V; ++j) other.v[j] = __shfl_xor(x[u].v[j], 32, kWave);
-        if (unit >= units) continue;
-        const uint32_t t = unit / total, local = unit % total;
-        const bool key = local >= q_heads;
-        const float inv = inv_lds[u];
-        const vecf<V>& w_own = key ? kw_own : qw_own;
-        const vecf<V>& w_par = key ? kw_par : qw_par;
-        const vecf<V> c = ldv<V>(cosine + static_cast<size_t>(t) * rope_stride + pair);
-        const vecf<V> s = ldv<V>(sine + static_cast<size_t>(t) * rope_stride + pair);
-        vecf<V> y;
-#pragma unroll
-        for (int j = 0; j < V; ++j) {
-            const float own = x[u].v[j] * inv * w_own.v[j];
-            const float par = other.v[j] * inv * w_par.v[j];
-            // low lanes hold x0 (own) and receive x1; high lanes the reverse
-            const float x0 = low ? own : par;
-            const float x1 = low ? par : own;
-            y.v[j] = low ? x0 * c.v[j] - x1 * s.v[j] : x0 * s.v[j] + x1 * c.v[j];
-        }
-        float* dst = key ? k_out + static_cast<size_t>(t) * D
-                         : q_out + (static_cast<size_t>(t) * q_heads + local) * D;
-        stv<V>(dst + col, y);
-    }
-}
-
-// Token engine (sequential order, the default for head_dim = 128*P): one
-// wavefront per token covers its q_heads Q rows and the optional K row
-// (U = q_heads + has_key <= MAXU units).  Lane l owns RoPE pairs
+// Token engine (head_dim 64 or 128 P): a wavefront covers units of one token,
+// its Q rows and the optional K row after them.  Lane l owns RoPE pairs
 // [l*P, l*P + P) of every unit and keeps both halves x[p] and x[p + d/2] in
 // registers, so the rotation needs no cross-lane exchange; the token's
-// cos/sin row and the four weight slices are loaded once per wavefront.
-// Loads are straight-line (units past U are clamped to a valid duplicate
-// address, never stored) and nontemporal; squares go to LDS and lane u folds
-// unit u in index order (bit-identical to the CPU composition
+// cos/sin row and the four weight slices are loaded once per wavefront.  At
+// head_dim 64 a register row holds two units (HPR = 2), one in each half of
+// the wavefront.  Loads are straight-line (units past the last are clamped to
+// a valid duplicate address, never stored) and nontemporal; squares go to LDS
+// and lane u folds unit u in index order (bit-identical to the CPU composition
 // rms_norm -> rope).  Every unit is fully read before it is written, so
 // q_out == q and k_out == k are allowed.
+__device__ __forceinline__ float half_wave_sum_tree_f32(float v) {  // wave_sum_tree_f32's steps inside each 32 lanes
+    v = v + dpp_f32<0xb1, 0xf, false>(v);
+    v = v + dpp_f32<0x4e, 0xf, false>(v);
+    v = v + dpp_f32<0x141, 0xf, false>(v);
+    v = v + dpp_f32<0x140, 0xf, false>(v);
+    return v + __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), 0x401f));
+}
+
 template <int P>
 struct pvec {
     float v[P];
@@ -246,99 +100,81 @@ __device__ __forceinline__ void sq_p(float* dst, const pvec<P>& x) {
     for (int j = 0; j < P; ++j) dst[j] = x.v[j] * x.v[j];
 }
 
-// TPW tokens per wavefront (tokens w and w + G, G = the grid's wavefront
-// count) and WPG wavefronts per workgroup; each wavefront uses its own LDS
-// region, so the handoff between the lanes that square and the lanes that
-// fold is a wavefront-scope fence, not a workgroup barrier.  SPLIT: a
-// token's units are spread over ceil(units / MAXU) consecutive wavefronts,
-// MAXU each (TPW = 1).  SEQ = false (ATLAS_REDUCTION_WIDE): each unit's sum
-// of squares is a wavefront tree sum of the lanes' partial sums instead of
-// the in-order fold (no LDS), tolerance-level against the CPU operator.
+// MAXU register rows of HPR units per wavefront, WPG wavefronts per
+// workgroup; each wavefront uses its own LDS region, so the handoff between
+// the lanes that square and the lanes that fold is a wavefront-scope fence,
+// not a workgroup barrier.  SPLIT: a token's units are spread over
+// consecutive wavefronts, MAXU HPR each; otherwise one wavefront has them all.
+// SEQ = false (ATLAS_REDUCTION_WIDE): each unit's sum of squares is a tree sum
+// of the lanes' partial sums instead of the in-order fold (no LDS),
+// tolerance-level against the CPU operator.
 // Parameter order: what the first loads' addresses need (the counts, the
 // rows, cos/sin) and epsilon fill the first 56 bytes, which arrive in SGPRs
 // at wave launch (kernarg preload); the weights and outputs, needed only
 // after the fold, follow.
-template <int P, int MAXU, int TPW, int WPG, bool SPLIT = false, bool SEQ = true>
+template <int P, int HPR, int MAXU, int WPG, bool SPLIT, bool SEQ>
 __global__ __launch_bounds__(64 * WPG) void qk_norm_rope_token_kernel(
     uint32_t tokens, uint32_t q_heads, uint32_t has_key, uint32_t rope_stride, const float* q, const float* k,
     const float* cosine, const float* sine, float epsilon, const float* q_weight, const float* k_weight,
     float* q_out, float* k_out) {
-    constexpr uint32_t HALF = 64 * P;
+    constexpr uint32_t kLanes = 64 / HPR;  // lanes of one head row
+    constexpr uint32_t HALF = kLanes * P;
     constexpr uint32_t D = 2 * HALF;
     constexpr uint32_t STRIDE = D + 4;
+    constexpr uint32_t kUnits = MAXU * HPR;  // a wavefront's units
     // head_dim 256 with one unit per wavefront: the unit's sum by candidate
     // segments (head_fold_candidates), from a padded copy of its squares
     // (float f at f + 4 (f / 64), 68 float4)
-    constexpr bool kCand = SEQ && D == 256 && TPW == 1 && MAXU == 1;
-    constexpr uint32_t kLds = kCand ? 272 : (SEQ ? TPW * MAXU * STRIDE : 4);
+    constexpr bool kCand = SEQ && D == 256 && kUnits == 1;
+    constexpr uint32_t kLds = kCand ? 272 : (SEQ ? kUnits * STRIDE : 4);
     __shared__ __align__(16) float sq_all[WPG][kLds];
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t wave = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6));
     float* sq = sq_all[wave];
-    static_assert(!SPLIT || TPW == 1, "a split token is one wavefront's only token");
     const uint32_t total = q_heads + has_key;
     const uint32_t wv = blockIdx.x * WPG + wave;
-    const uint32_t parts = SPLIT ? (total + MAXU - 1) / MAXU : 1u;
-    const uint32_t w0 = SPLIT ? wv / parts : wv;
-    const uint32_t ubase = SPLIT ? (wv - w0 * parts) * MAXU : 0u;  // the wavefront's first unit
-    const uint32_t G = gridDim.x * WPG;
-    if (w0 >= tokens) return;  // wavefront-uniform
-    const uint32_t p0 = lane * P;
-    uint32_t tok[TPW];
-    uint32_t ntok = 0;
-#pragma unroll
-    for (int i = 0; i < TPW; ++i) {
-        tok[i] = w0 + i * G;
-        ntok += tok[i] < tokens ? 1u : 0u;
-    }
+    const uint32_t parts = SPLIT ? (total + kUnits - 1) / kUnits : 1u;
+    const uint32_t t = SPLIT ? wv / parts : wv;
+    const uint32_t ubase = SPLIT ? (wv - t * parts) * kUnits : 0u;  // the wavefront's first unit
+    if (t >= tokens) return;  // wavefront-uniform
+    const uint32_t hs = HPR == 1 ? 0u : lane / kLanes;  // the lane's head of each register row
+    const uint32_t p0 = (HPR == 1 ? lane : lane % kLanes) * P;
 
-    pvec<P> lo[TPW][MAXU], hi[TPW][MAXU];
+    pvec<P> lo[MAXU], hi[MAXU];
 #pragma unroll
-    for (int i = 0; i < TPW; ++i) {
-        const uint32_t t = min(tok[i], tokens - 1);
-#pragma unroll
-        for (int u = 0; u < MAXU; ++u) {
-            const uint32_t uu = min(ubase + u, total - 1);
-            const float* src = uu >= q_heads ? k + static_cast<size_t>(t) * D
-                                             : q + (static_cast<size_t>(t) * q_heads + uu) * D;
-            lo[i][u] = ld_p<P, true>(src + p0);
-            hi[i][u] = ld_p<P, true>(src + HALF + p0);
-        }
+    for (int u = 0; u < MAXU; ++u) {
+        const uint32_t uu = min(ubase + u * HPR + hs, total - 1);
+        const float* src = uu >= q_heads ? k + static_cast<size_t>(t) * D
+                                         : q + (static_cast<size_t>(t) * q_heads + uu) * D;
+        lo[u] = ld_p<P, true>(src + p0);
+        hi[u] = ld_p<P, true>(src + HALF + p0);
     }
-    pvec<P> cs[TPW], sn[TPW];
-#pragma unroll
-    for (int i = 0; i < TPW; ++i) {
-        const size_t tb = static_cast<size_t>(min(tok[i], tokens - 1)) * rope_stride + p0;
-        cs[i] = ld_p<P, false>(cosine + tb);
-        sn[i] = ld_p<P, false>(sine + tb);
-    }
+    const size_t tb = static_cast<size_t>(t) * rope_stride + p0;
+    const pvec<P> c = ld_p<P, false>(cosine + tb);
+    const pvec<P> s = ld_p<P, false>(sine + tb);
     const pvec<P> qwl = ld_p<P, false>(q_weight + p0), qwh = ld_p<P, false>(q_weight + HALF + p0);
     const float* kw = has_key ? k_weight : q_weight;
     const pvec<P> kwl = ld_p<P, false>(kw + p0), kwh = ld_p<P, false>(kw + HALF + p0);
 
-    // lane i * MAXU + u holds the sum of squares of unit u of the
-    // wavefront's token i
+    // lane u holds the sum of squares of the wavefront's unit u
     float sum = 0.0f;
-    const uint32_t li = lane / MAXU, lu = lane - li * MAXU;
-    const bool folds = li < ntok && ubase + lu < total;
+    const bool folds = lane < kUnits && ubase + lane < total;
     if constexpr (kCand) {
         // lane l's values p0, p0 + 1 (P = 2) and HALF + p0, ...: each pair
         // inside one 64-float segment
-        sq_p<P>(sq + p0 + 4 * (p0 / 64), lo[0][0]);
-        sq_p<P>(sq + HALF + p0 + 4 * ((HALF + p0) / 64), hi[0][0]);
+        sq_p<P>(sq + p0 + 4 * (p0 / 64), lo[0]);
+        sq_p<P>(sq + HALF + p0 + 4 * ((HALF + p0) / 64), hi[0]);
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        const float t = head_fold_candidates(reinterpret_cast<const f32x4*>(sq), lane);
-        sum = lane == 0 ? t : sum;
+        const float f = head_fold_candidates(reinterpret_cast<const f32x4*>(sq), lane);
+        sum = lane == 0 ? f : sum;
     } else if constexpr (SEQ) {
 #pragma unroll
-        for (int i = 0; i < TPW; ++i)
-#pragma unroll
-            for (int u = 0; u < MAXU; ++u) {
-                sq_p<P>(sq + (i * MAXU + u) * STRIDE + p0, lo[i][u]);
-                sq_p<P>(sq + (i * MAXU + u) * STRIDE + HALF + p0, hi[i][u]);
-            }
+        for (int u = 0; u < MAXU; ++u) {
+            sq_p<P>(sq + (u * HPR + hs) * STRIDE + p0, lo[u]);
+            sq_p<P>(sq + (u * HPR + hs) * STRIDE + HALF + p0, hi[u]);
+        }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -346,130 +182,144 @@ __global__ __launch_bounds__(64 * WPG) void qk_norm_rope_token_kernel(
         if (folds) {
             const f32x4* row = reinterpret_cast<const f32x4*>(sq + lane * STRIDE);
 #pragma unroll
-            for (uint32_t c = 0; c < D / 4; c += 64)
-                sum = fold_lds_chunk(row + c, D / 4 - c < 64 ? D / 4 - c : 64, sum);
+            for (uint32_t f = 0; f < D / 4; f += 64)
+                sum = fold_lds_chunk(row + f, D / 4 - f < 64 ? D / 4 - f : 64, sum);
         }
     } else {
         (void)sq;
 #pragma unroll
-        for (int i = 0; i < TPW; ++i)
+        for (int u = 0; u < MAXU; ++u) {
+            float part = 0.0f;
 #pragma unroll
-            for (int u = 0; u < MAXU; ++u) {
-                float part = 0.0f;
+            for (int j = 0; j < P; ++j) part = part + lo[u].v[j] * lo[u].v[j];
 #pragma unroll
-                for (int j = 0; j < P; ++j) part = part + lo[i][u].v[j] * lo[i][u].v[j];
-#pragma unroll
-                for (int j = 0; j < P; ++j) part = part + hi[i][u].v[j] * hi[i][u].v[j];
-                const float t = wave_sum_tree_f32(part);
-                sum = lane == static_cast<uint32_t>(i * MAXU + u) ? t : sum;
+            for (int j = 0; j < P; ++j) part = part + hi[u].v[j] * hi[u].v[j];
+            if constexpr (HPR == 1) {
+                const float f = wave_sum_tree_f32(part);
+                sum = lane == static_cast<uint32_t>(u) ? f : sum;
+            } else {
+                const float f = half_wave_sum_tree_f32(part);
+                sum = lane == static_cast<uint32_t>(2 * u) ? readlane_f32(f, 0) : sum;
+                sum = lane == static_cast<uint32_t>(2 * u + 1) ? readlane_f32(f, 32) : sum;
             }
+        }
     }
     const float inv = folds ? inverse_rms(sum, static_cast<float>(D), epsilon) : 0.0f;
 
 #pragma unroll
-    for (int i = 0; i < TPW; ++i) {
-        if (static_cast<uint32_t>(i) >= ntok) break;
-        const uint32_t t = tok[i];
-        const pvec<P>& c = cs[i];
-        const pvec<P>& s = sn[i];
+    for (int u = 0; u < MAXU; ++u) {
+        const uint32_t unit = ubase + u * HPR + hs;
+        if (unit < total) {
+            // readlane reads the lane's register whatever lanes are active
+            float iu = readlane_f32(inv, u * HPR);
+            if (HPR == 2) iu = hs ? readlane_f32(inv, u * HPR + 1) : iu;
+            const bool key = unit >= q_heads;
+            pvec<P> ol, oh;
 #pragma unroll
-        for (int u = 0; u < MAXU; ++u) {
-            if (ubase + u < total) {
-                const float iu = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(inv), i * MAXU + u));
-                const bool key = ubase + u >= q_heads;
-                pvec<P> ol, oh;
-#pragma unroll
-                for (int j = 0; j < P; ++j) {
-                    const float wl = key ? kwl.v[j] : qwl.v[j];
-                    const float wh = key ? kwh.v[j] : qwh.v[j];
-                    const float x0 = lo[i][u].v[j] * iu * wl;
-                    const float x1 = hi[i][u].v[j] * iu * wh;
-                    ol.v[j] = x0 * c.v[j] - x1 * s.v[j];
-                    oh.v[j] = x0 * s.v[j] + x1 * c.v[j];
-                }
-                float* dst = key ? k_out + static_cast<size_t>(t) * D
-                                 : q_out + (static_cast<size_t>(t) * q_heads + ubase + u) * D;
-                st_p<P>(dst + p0, ol);
-                st_p<P>(dst + HALF + p0, oh);
+            for (int j = 0; j < P; ++j) {
+                const float wl = key ? kwl.v[j] : qwl.v[j];
+                const float wh = key ? kwh.v[j] : qwh.v[j];
+                const float x0 = lo[u].v[j] * iu * wl;
+                const float x1 = hi[u].v[j] * iu * wh;
+                ol.v[j] = x0 * c.v[j] - x1 * s.v[j];
+                oh.v[j] = x0 * s.v[j] + x1 * c.v[j];
             }
+            float* dst = key ? k_out + static_cast<size_t>(t) * D
+                             : q_out + (static_cast<size_t>(t) * q_heads + unit) * D;
+            st_p<P>(dst + p0, ol);
+            st_p<P>(dst + HALF + p0, oh);
         }
     }
 }
 
-template <int P, int TPW, int WPG, bool SEQ>
-hipError_t launch_qk_token_cfg(hipStream_t s, const float* q, const float* k, const float* qw, const float* kw,
-                               const float* c, const float* sn, float* qo, float* ko, uint32_t tokens,
-                               uint32_t q_heads, uint32_t has_key, uint32_t rope_stride, float eps) {
-    const uint32_t total = q_heads + has_key;
-    const uint32_t waves = (tokens + TPW - 1) / TPW;
-    const dim3 grid((waves + WPG - 1) / WPG);
-#define ATLAS_QK_CASE(U)                                                                                          \
-    if (total <= U) {                                                                                             \
-        hipLaunchKernelGGL((qk_norm_rope_token_kernel<P, U, TPW, WPG, false, SEQ>), grid, dim3(64 * WPG), 0, s,      \
-                           tokens, q_heads, has_key, rope_stride, q, k, c, sn, eps, qw, kw, qo, ko);            \
-        return hipGetLastError();                                                                                 \
-    }
-    ATLAS_QK_CASE(1)
-    ATLAS_QK_CASE(2)
-    ATLAS_QK_CASE(4)
-    ATLAS_QK_CASE(8)
-    ATLAS_QK_CASE(9)
-    ATLAS_QK_CASE(12)
-    ATLAS_QK_CASE(16)
-#undef ATLAS_QK_CASE
-    return hipErrorInvalidValue;
-}
-
-// A token's units over ceil(units / U) wavefronts, one wavefront per workgroup.
-template <int P, int U, bool SEQ>
-hipError_t launch_qk_split(hipStream_t s, const float* q, const float* k, const float* qw, const float* kw,
-                           const float* c, const float* sn, float* qo, float* ko, uint32_t tokens, uint32_t q_heads,
-                           uint32_t has_key, uint32_t rope_stride, float eps) {
-    const uint32_t total = q_heads + has_key;
-    const uint64_t waves = static_cast<uint64_t>(tokens) * ((total + U - 1) / U);
-    if (waves > 0x7fffffffu) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((qk_norm_rope_token_kernel<P, U, 1, 1, true, SEQ>), dim3(static_cast<uint32_t>(waves)), dim3(64), 0,
-                       s, tokens, q_heads, has_key, rope_stride, q, k, c, sn, eps, qw, kw, qo, ko);
+#define ATLAS_QK_PARAMS                                                                                            \
+    hipStream_t stream, const float *q, const float *k, const float *qw, const float *kw, const float *c,          \
+        const float *sn, float *qo, float *ko, uint32_t tokens, uint32_t q_heads, uint32_t has_key,                \
+        uint32_t rope_stride, float eps
+#define ATLAS_QK_ARGS stream, q, k, qw, kw, c, sn, qo, ko, tokens, q_heads, has_key, rope_stride, eps
+#define ATLAS_QK_LAUNCH(R, WPG, SPLIT, blocks)                                                                     \
+    hipLaunchKernelGGL((qk_norm_rope_token_kernel<P, HPR, R, WPG, SPLIT, SEQ>), dim3(blocks), dim3(64 * (WPG)), 0, \
+                       stream, tokens, q_heads, has_key, rope_stride, q, k, c, sn, eps, qw, kw, qo, ko);           \
     return hipGetLastError();
+
+// One wavefront per token (at most 16 units), WPG per workgroup.
+template <int P, int HPR, int WPG, bool SEQ>
+hipError_t launch_qk_token(ATLAS_QK_PARAMS) {
+    const uint32_t rows = (q_heads + has_key + HPR - 1) / HPR, blocks = (tokens + WPG - 1) / WPG;
+    if (rows <= 1) { ATLAS_QK_LAUNCH(1, WPG, false, blocks) }
+    if (rows <= 2) { ATLAS_QK_LAUNCH(2, WPG, false, blocks) }
+    if (rows <= 4) { ATLAS_QK_LAUNCH(4, WPG, false, blocks) }
+    if constexpr (HPR == 2) {
+        if (rows <= 5) { ATLAS_QK_LAUNCH(5, WPG, false, blocks) }
+        ATLAS_QK_LAUNCH(8, WPG, false, blocks)
+    } else {
+        if (rows <= 8) { ATLAS_QK_LAUNCH(8, WPG, false, blocks) }
+        if (rows <= 9) { ATLAS_QK_LAUNCH(9, WPG, false, blocks) }
+        if (rows <= 12) { ATLAS_QK_LAUNCH(12, WPG, false, blocks) }
+        ATLAS_QK_LAUNCH(16, WPG, false, blocks)
+    }
 }
 
-// Wavefronts per token by token count.  A wavefront folds its units' rows
-// in order (lane u, unit u), a chain of 2 * P * 64 adds whatever the unit
-// count, while its loads, squares and rotations grow with the units it
-// holds; few tokens leave most CUs idle, so below 768 tokens a token's
-// units are spread over several wavefronts.  Measured on MI355X (8 Q heads
-// + K, head_dim 256, per launch over rotating buffer sets):
-//   tokens     1 unit/wave  2 units  1 token/wave  4 tokens/workgroup
-//   256          4.80        4.81      5.46          6.10 us
-//   512          5.78        5.32      6.06          6.27
-//   1024         8.32        7.45      6.62          6.51
-//   1536        10.63        9.70      7.16          7.45
-//   2047        13.00       11.07      7.88          8.00
-// and at 4096 tokens 14.17 us with four wavefronts per workgroup against
-// 14.25-14.33 with one and 18.3 with two units per wavefront.  With one unit
-// per wavefront the unit's fold runs by candidate segments (head_dim 256),
-// which moves the first crossover: 256 tokens 3.87 against 4.08 us with two
-// units per wavefront, 384 4.31 against 4.39, 512 4.85 against 4.76, 767
-// 6.47 against 5.93.  In the C5 decode step (a graph of 35 launches): 256
-// tokens 3.59-3.60 us (3.86 with two units per wavefront, 4.72 with one
-// wavefront per token); one token 2.20-2.22 (2.55 with the in-order fold).
-template <int P, bool SEQ>
-hipError_t launch_qk_token_p(hipStream_t s, const float* q, const float* k, const float* qw, const float* kw,
-                             const float* c, const float* sn, float* qo, float* ko, uint32_t tokens,
-                             uint32_t q_heads, uint32_t has_key, uint32_t rope_stride, float eps) {
-    if (tokens >= 2048)
-        return launch_qk_token_cfg<P, 1, 4, SEQ>(s, q, k, qw, kw, c, sn, qo, ko, tokens, q_heads, has_key, rope_stride,
-                                            eps);
-    if (tokens >= 768)
-        return launch_qk_token_cfg<P, 1, 1, SEQ>(s, q, k, qw, kw, c, sn, qo, ko, tokens, q_heads, has_key, rope_stride,
-                                            eps);
-    if (tokens >= 512)
-        return launch_qk_split<P, 2, SEQ>(s, q, k, qw, kw, c, sn, qo, ko, tokens, q_heads, has_key, rope_stride, eps);
-    return launch_qk_split<P, 1, SEQ>(s, q, k, qw, kw, c, sn, qo, ko, tokens, q_heads, has_key, rope_stride, eps);
+// A token's units over several wavefronts, R register rows each, one
+// wavefront per workgroup.
+template <int P, int HPR, int R, bool SEQ>
+hipError_t launch_qk_split(ATLAS_QK_PARAMS) {
+    const uint32_t total = q_heads + has_key;
+    const uint64_t waves = static_cast<uint64_t>(tokens) * ((total + R * HPR - 1) / (R * HPR));
+    if (waves > 0x7fffffffu) return hipErrorInvalidValue;
+    ATLAS_QK_LAUNCH(R, 1, true, static_cast<uint32_t>(waves))
 }
 
-// Generic head_dim fallback (even head_dim not of the form 64*V): one wave
-// per unit, row staged in LDS.
+// Units per wavefront by the launch's units (tokens x heads).  A wavefront
+// folds its units' rows in order side by side (lane u, unit u), a chain of
+// head_dim adds whatever the unit count (64 and three selections for one unit
+// at head_dim 256, by candidate segments), while its loads, squares and
+// rotations grow with the units it holds: few units are spread over as many
+// wavefronts, many are gathered, up to a token's whole row of heads.
+// Measured on MI355X (us, graph of back-to-back launches over rotating
+// buffers; R = register rows per wavefront, two units each at head_dim 64;
+// "token" one wavefront per token; the last column the engine that took 17
+// and more heads, and head_dim 64, before):
+//   head_dim  units           R=1    R=2    R=4    token or R=9
+//   256       2304 (256 x 9)  3.69   3.78   4.34   4.74
+//             4352 (256 x 17) 4.44   4.47   4.61   5.35         10.8
+//             6912 (768 x 9)  6.10   5.23   5.23   5.73
+//             9000 (1000 x 9) 7.18   6.85   5.78   6.07
+//             13056 (768 x 17) 8.99  8.88   7.56   6.73         14.9
+//             34816 (2048 x 17) 19.2 16.8   16.0   13.5         22.9
+//   512       1152 (128 x 9)  4.48   5.07   5.32   5.93
+//             4352 (256 x 17) 7.75   6.29   6.34   7.59         12.8
+//             8704 (512 x 17) 11.8   10.4   9.05   8.81         16.8
+//   128       1152 (128 x 9)  2.96   3.03   3.30   3.91
+//             8704 (512 x 17) 5.13   4.19   4.21   4.70         9.37
+//             17000 (1000 x 17) 7.40 6.58   5.24   5.49         12.2
+//   64        1280 (256 x 5)  2.50   2.54   2.64   2.79         3.26
+//             9000 (1000 x 9) 3.81   3.45   3.65   3.97         5.95
+//             36864 (4096 x 9) 7.56  6.79   6.97   5.30         15.9
+// From 2048 tokens there are wavefronts enough with one per token, whatever
+// its units ([2048, 4 + 1, 256] 6.09 us against 7.44 with four units each),
+// four tokens per workgroup ([4096, 8 + 1, 256] 14.17 us against 14.25-14.33
+// with one); the tree sum has no chain to spread, so it takes them from 768
+// tokens ([1000, 8 + 1, 256] 5.66 against 6.15).
+template <int P, int HPR, bool SEQ>
+hipError_t launch_qk_p(ATLAS_QK_PARAMS) {
+    constexpr uint32_t kOne = P == 4 ? 1800 : (P == 2 ? 4500 : 2500);
+    constexpr uint32_t kTwo = P == 4 ? 5000 : (P == 2 ? 7000 : 10000);
+    constexpr uint32_t kFour = P == 4 ? 8500 : (P == 2 ? 11000 : 20000);
+    const uint32_t total = q_heads + has_key;
+    const uint64_t units = static_cast<uint64_t>(tokens) * total;
+    if (total <= 16 && tokens >= 2048) return launch_qk_token<P, HPR, 4, SEQ>(ATLAS_QK_ARGS);
+    if (total <= 16 && tokens >= 768 && !SEQ) return launch_qk_token<P, HPR, 1, SEQ>(ATLAS_QK_ARGS);
+    if (units < kOne) return launch_qk_split<P, HPR, 1, SEQ>(ATLAS_QK_ARGS);
+    if (units < kTwo) return launch_qk_split<P, HPR, 2, SEQ>(ATLAS_QK_ARGS);
+    if (units < kFour) return launch_qk_split<P, HPR, 4, SEQ>(ATLAS_QK_ARGS);
+    if (total > 16) return launch_qk_split<P, HPR, 9, SEQ>(ATLAS_QK_ARGS);
+    return launch_qk_token<P, HPR, 1, SEQ>(ATLAS_QK_ARGS);
+}
+#undef ATLAS_QK_LAUNCH
+
+// Generic fallback (other even head_dims, unaligned operands): one wave per
+// unit, row staged in LDS.
 __global__ __launch_bounds__(64) void qk_norm_rope_generic_kernel(
     const float* q, const float* k, const float* q_weight, const float* k_weight,
     const float* cosine, const float* sine, float* q_out, float* k_out, uint32_t tokens,
@@ -650,22 +500,6 @@ __global__ __launch_bounds__(256) void rope_interleaved_kernel(const float* x, c
 
 bool aligned(const void* p, uintptr_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; }
 
-template <int V, int UNITS>
-hipError_t launch_qk(hipStream_t s, bool seq, const float* q, const float* k, const float* qw,
-                     const float* kw, const float* c, const float* sn, float* qo, float* ko,
-                     uint32_t tokens, uint32_t q_heads, uint32_t has_key, uint32_t rope_stride,
-                     float eps) {
-    const uint32_t units = tokens * (q_heads + has_key);
-    const dim3 grid((units + UNITS - 1) / UNITS);
-    if (seq)
-        hipLaunchKernelGGL((qk_norm_rope_kernel<V, UNITS, true>), grid, dim3(kWave), 0, s, q, k, qw,
-                           kw, c, sn, qo, ko, tokens, q_heads, has_key, rope_stride, eps);
-    else
-        hipLaunchKernelGGL((qk_norm_rope_kernel<V, UNITS, false>), grid, dim3(kWave), 0, s, q, k, qw,
-                           kw, c, sn, qo, ko, tokens, q_heads, has_key, rope_stride, eps);
-    return hipGetLastError();
-}
-
 }  // namespace
 
 hipError_t launch_qk_norm_rope_f32(hipStream_t stream, Reduction red, const float* q, const float* k,
@@ -677,47 +511,26 @@ hipError_t launch_qk_norm_rope_f32(hipStream_t stream, Reduction red, const floa
     // the rotation after the norm can cancel, so only ATLAS_REDUCTION_WIDE
     // reorders the sum of squares here; kAuto keeps the sequential fold
     const bool seq = red != kWide;
-    // Token engine: head_dim = 128*P, at most 16 units per token, operands
-    // and per-token cos/sin rows aligned to P floats; the in-order fold, or
-    // under WIDE the wavefront tree sum.  Measured on MI355X (C5 decode, 8 Q
-    // heads + K, head_dim 256): WIDE took 12.7 us at 256 tokens and 9.5 at
-    // one token on the unit engine below, which puts 16 units on one
-    // wavefront one after another.
-    {
-        const uint32_t P = head_dim / 128;
-        const uintptr_t pa = 4u * (P == 0 ? 1 : P) > 16 ? 16 : 4u * (P == 0 ? 1 : P);
-        const bool ok = head_dim % 128 == 0 && (P == 1 || P == 2 || P == 4) && q_heads + has_key <= 16 &&
-                        q_heads + has_key > 0 && aligned(q, pa) && aligned(q_out, pa) && aligned(q_weight, pa) &&
-                        aligned(cosine, pa) && aligned(sine, pa) && rope_stride % P == 0 &&
-                        (!has_key || (aligned(k, pa) && aligned(k_out, pa) && aligned(k_weight, pa)));
-        if (ok) {
-#define ATLAS_QK_TOKEN(PP)                                                                                        \
-    return seq ? launch_qk_token_p<PP, true>(stream, q, k, q_weight, k_weight, cosine, sine, q_out, k_out, tokens, \
-                                             q_heads, has_key, rope_stride, epsilon)                                 \
-               : launch_qk_token_p<PP, false>(stream, q, k, q_weight, k_weight, cosine, sine, q_out, k_out,         \
-                                              tokens, q_heads, has_key, rope_stride, epsilon);
-            if (P == 1) ATLAS_QK_TOKEN(1)
-            if (P == 2) ATLAS_QK_TOKEN(2)
-            ATLAS_QK_TOKEN(4)
-#undef ATLAS_QK_TOKEN
-        }
-    }
-    // Unit engine: head_dim = 64*V, 16-byte aligned operands (8-byte for V=2),
-    // and per-token cos/sin rows aligned to the vector width.
-    const uintptr_t va = head_dim == 128 ? 8 : 16;
-    const bool vec_ok = (head_dim == 128 || head_dim == 256 || head_dim == 512) && aligned(q, va) &&
-                        aligned(q_out, va) && aligned(q_weight, va) && aligned(cosine, va) &&
-                        aligned(sine, va) && (rope_stride % (head_dim / 64)) == 0 &&
-                        (!has_key || (aligned(k, va) && aligned(k_out, va) && aligned(k_weight, va)));
-    if (vec_ok) {
-        if (head_dim == 256)
-            return launch_qk<4, 16>(stream, seq, q, k, q_weight, k_weight, cosine, sine, q_out, k_out,
-                                    tokens, q_heads, has_key, rope_stride, epsilon);
-        if (head_dim == 512)
-            return launch_qk<8, 8>(stream, seq, q, k, q_weight, k_weight, cosine, sine, q_out, k_out,
-                                   tokens, q_heads, has_key, rope_stride, epsilon);
-        return launch_qk<2, 16>(stream, seq, q, k, q_weight, k_weight, cosine, sine, q_out, k_out,
-                                tokens, q_heads, has_key, rope_stride, epsilon);
+    // Token engine: head_dim 64 or 128*P, operands and per-token cos/sin rows
+    // aligned to P floats; the in-order fold, or under WIDE the wavefront
+    // tree sum.
+    const uint32_t P = head_dim == 64 ? 1 : head_dim / 128;
+    const uintptr_t pa = 4u * (P == 0 ? 1 : P);
+    const bool ok = (head_dim == 64 || (head_dim % 128 == 0 && (P == 1 || P == 2 || P == 4))) && aligned(q, pa) &&
+                    aligned(q_out, pa) && aligned(q_weight, pa) && aligned(cosine, pa) && aligned(sine, pa) &&
+                    rope_stride % P == 0 &&
+                    (!has_key || (aligned(k, pa) && aligned(k_out, pa) && aligned(k_weight, pa)));
+    if (ok) {
+        const float *qw = q_weight, *kw = k_weight, *c = cosine, *sn = sine;
+        float *qo = q_out, *ko = k_out;
+        const float eps = epsilon;
+#define ATLAS_QK_P(PP, HPR) \
+    return seq ? launch_qk_p<PP, HPR, true>(ATLAS_QK_ARGS) : launch_qk_p<PP, HPR, false>(ATLAS_QK_ARGS);
+        if (head_dim == 64) { ATLAS_QK_P(1, 2) }
+        if (P == 1) { ATLAS_QK_P(1, 1) }
+        if (P == 2) { ATLAS_QK_P(2, 1) }
+        ATLAS_QK_P(4, 1)
+#undef ATLAS_QK_P
     }
     const uint32_t units = tokens * (q_heads + has_key);
     hipLaunchKernelGGL(qk_norm_rope_generic_kernel, dim3(units), dim3(kWave),
