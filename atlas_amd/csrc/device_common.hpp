@@ -77,6 +77,7 @@ __device__ __forceinline__ float pow2i(int k) {  // 2^k, k in [-126, 127]
 // branch per element costs an exec-mask round trip per wave and measured
 // ~10 % of GeGLU's time).  exp_small_f32 is the form for arguments known to
 // lie in (-87, 87), where no special range applies.
+template <bool CLAMP = true>
 __device__ __forceinline__ float exp_reduced(float x, int& n) {
     const float log2e = 1.44269502162933349609375f;
     const float ln2_hi = 0.693359375f;
@@ -85,8 +86,9 @@ __device__ __forceinline__ float exp_reduced(float x, int& n) {
     // every input.  One v_med3 (instead of a min and a max): the two clamps
     // differ only for NaN, whose result stays NaN through r either way, and
     // the clamp only acts for |x| > 138, whose results every caller selects
-    // away.
-    const float fn = __builtin_amdgcn_fmed3f(floorf(__builtin_fmaf(x, log2e, 0.5f)), -200.0f, 200.0f);
+    // away (CLAMP = false: |x| < 87, where it never acts).
+    const float fl = floorf(__builtin_fmaf(x, log2e, 0.5f));
+    const float fn = CLAMP ? __builtin_amdgcn_fmed3f(fl, -200.0f, 200.0f) : fl;
     n = static_cast<int>(fn);
     const float r = __builtin_fmaf(-fn, ln2_lo, __builtin_fmaf(-fn, ln2_hi, x));
     float p = 1.0f / 5040.0f;
@@ -190,6 +192,26 @@ __device__ __forceinline__ float tanh_exp_abs(float a) {
     return 1.0f - fdiv_rn(2.0f, e + 1.0f);
 }
 __device__ __forceinline__ bool tanh_series_range(float a) { return a < 0.625f; }
+
+// tanh_exp_abs for a >= 0.625 with the quotient by D::div and no special
+// ranges: a is clamped at 40, where 2/(e^{2a} + 1) is far below half an ulp
+// of 1 and the result is 1 as it is above (e^{2a} then stays in the range
+// where exp_small_f32 is exp_f32; inf included).  NaN gives 1: callers select
+// it away.  A GPU test runs it on every a of its domain against tanh_exp_abs.
+template <class D>
+__device__ __forceinline__ float tanh_exp_abs_with(float a) {
+    int n;
+    const float p = exp_reduced<false>(2.0f * fminf(a, 40.0f), n);
+    return 1.0f - D::div(2.0f, __builtin_ldexpf(p, n) + 1.0f);
+}
+// div_inrange without its sign step, for positive operands.
+struct DivPositive {
+    __device__ static float div(float a, float b) {
+        const float r = __builtin_amdgcn_rcpf(b);
+        const float q0 = a * r;
+        return __builtin_fmaf(__builtin_fmaf(-q0, b, a), r, q0);
+    }
+};
 
 // x / (1 + e^-x)   (kernels.metal:27-36)
 __device__ __forceinline__ float silu_f32(float x) { return fdiv_rn(x, 1.0f + exp_f32(-x)); }

@@ -17,6 +17,9 @@
 //                        arguments; |v| >= 10 selects +-1 after the quotient)
 //   1  gelu_finite_with: every x whose GELU argument is finite
 //   2  silu_small_with:  every x with |x| < 87 (silu_lanes' branch)
+//   3  tanh_exp_abs_with<DivPositive> against tanh_exp_abs (IEEE division, the
+//      whole exponential range): every a in [0.625, inf] (softcap_lanes); the
+//      planted product beside it, the sign step does not apply
 #include "device_common.hpp"
 
 #include <stdint.h>
@@ -39,6 +42,7 @@ template <int DOMAIN, class D>
 __device__ __forceinline__ float eval(float x) {
     if (DOMAIN == 0) return tanh_with<D>(x);
     if (DOMAIN == 1) return gelu_finite_with<D>(x, gelu_argument(x));
+    if (DOMAIN == 3) return tanh_exp_abs_with<D>(x);
     return silu_small_with<D>(x);
 }
 
@@ -46,6 +50,7 @@ template <int DOMAIN>
 __device__ __forceinline__ bool in_domain(float x) {
     if (DOMAIN == 0) return __builtin_fabsf(x) < __builtin_inff();
     if (DOMAIN == 1) return __builtin_fabsf(gelu_argument(x)) < __builtin_inff();
+    if (DOMAIN == 3) return x >= 0.625f;
     return __builtin_fabsf(x) < 87.0f;
 }
 
@@ -59,9 +64,9 @@ __global__ __launch_bounds__(256) void enumerate_kernel(unsigned long long* coun
     for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < (1ull << 32); i += stride) {
         const float x = __uint_as_float(static_cast<uint32_t>(i));
         if (!in_domain<DOMAIN>(x)) continue;
-        const uint32_t ref = __float_as_uint(eval<DOMAIN, DivIeee>(x));
+        const uint32_t ref = __float_as_uint(DOMAIN == 3 ? tanh_exp_abs(x) : eval<DOMAIN, DivIeee>(x));
         ++n;
-        bad += __float_as_uint(eval<DOMAIN, DivInRange>(x)) != ref;
+        bad += __float_as_uint(DOMAIN == 3 ? eval<DOMAIN, DivPositive>(x) : eval<DOMAIN, DivInRange>(x)) != ref;
         bad_product += __float_as_uint(eval<DOMAIN, DivProduct>(x)) != ref;
         bad_sign += __float_as_uint(eval<DOMAIN, DivNoSign>(x)) != ref;
     }
@@ -74,11 +79,11 @@ __global__ __launch_bounds__(256) void enumerate_kernel(unsigned long long* coun
 }  // namespace
 }  // namespace atlas
 
-// Runs the enumeration of `domain` (0 tanh, 1 GELU, 2 SiLU) on the current
+// Runs the enumeration of `domain` (0 tanh, 1 GELU, 2 SiLU, 3 soft cap) on the current
 // device and writes the four counts to host memory.  Returns 0, -1 for an
 // unknown domain, or the HIP error code.
 extern "C" int atlas_division_check(int domain, uint64_t* counts) {
-    if (domain < 0 || domain > 2 || counts == nullptr) return -1;
+    if (domain < 0 || domain > 3 || counts == nullptr) return -1;
     unsigned long long* d = nullptr;
     hipError_t e = hipMalloc(&d, 4 * sizeof(unsigned long long));
     if (e != hipSuccess) return static_cast<int>(e);
@@ -88,6 +93,7 @@ extern "C" int atlas_division_check(int domain, uint64_t* counts) {
         if (domain == 0) hipLaunchKernelGGL(atlas::enumerate_kernel<0>, grid, block, 0, 0, d);
         if (domain == 1) hipLaunchKernelGGL(atlas::enumerate_kernel<1>, grid, block, 0, 0, d);
         if (domain == 2) hipLaunchKernelGGL(atlas::enumerate_kernel<2>, grid, block, 0, 0, d);
+        if (domain == 3) hipLaunchKernelGGL(atlas::enumerate_kernel<3>, grid, block, 0, 0, d);
         e = hipGetLastError();
     }
     if (e == hipSuccess) e = hipDeviceSynchronize();

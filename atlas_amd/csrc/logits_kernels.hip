@@ -43,36 +43,119 @@ __device__ __forceinline__ uint64_t argmax_key(float v, uint32_t index) {
 
 __device__ __forceinline__ uint64_t max_u64(uint64_t a, uint64_t b) { return a > b ? a : b; }
 
-// cap * tanh(v / cap) for the values of one lane.  The series range is
-// evaluated for every value; the exponential range only when some lane of
-// the wavefront needs it (a wave-uniform branch), then selected per value.
-template <int N>
-__device__ __forceinline__ void softcap_lanes(float (&v)[N], float cap) {
-    float t[N], a[N], r[N];
-    bool need_exp = false;
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-        t[i] = fdiv_rn(v[i], cap);
-        a[i] = __builtin_fabsf(t[i]);
-        need_exp = need_exp || !tanh_series_range(a[i]);
-        r[i] = tanh_series_abs(a[i]);
-    }
-    if (__builtin_amdgcn_ballot_w64(need_exp) != 0) {
-#pragma unroll
-        for (int i = 0; i < N; ++i) {
-            const float big = tanh_exp_abs(a[i]);
-            r[i] = tanh_series_range(a[i]) ? r[i] : big;
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < N; ++i) v[i] = cap * __builtin_copysignf(r[i], t[i]);
+// The cap and what a wavefront's plain values need of it: rcp = RN(1 / cap).
+struct SoftCap {
+    float cap, rcp;
+    bool plain;  // cap in [2^-20, 2^20]
+};
+
+__device__ __forceinline__ SoftCap soft_cap(float cap) {
+    return {cap, fdiv_rn(1.0f, cap), cap >= 0x1p-20f && cap <= 0x1p20f};
 }
 
-// Reduce a workgroup's key and publish it: the row's index when the row has
-// one workgroup, otherwise the workgroup's slot of the workspace.
+// cap * tanh(v / cap) for the values of one lane, with the bits of the IEEE
+// steps (fdiv_rn, tanh_series_abs, tanh_exp_abs) throughout.  The series is
+// evaluated for every value; the exponential only when some lane of the
+// wavefront needs it (a wave-uniform branch), then selected per value.  Bound
+// by this arithmetic where logits reach the exponential (|v| >= 0.625 cap),
+// so wavefronts whose |v| all lie in [2^-70, 2^60] -- ordinary logits; an
+// exact zero, an infinity or a NaN row sends the wavefront to the full form --
+// take shorter divisions:
+//  * v / cap: q0 = v rcp is within 1.5 ulp of the quotient; q1 = fma(v - q0
+//    cap, rcp, q0) within half an ulp and a few 2^-22 of one, so faithful; and
+//    q2 = fma(v - q1 cap, rcp, q1), with the residual exact (no operand or
+//    product comes near the subnormals) and rcp correctly rounded, is the
+//    correctly rounded quotient (Markstein 1990).  Five operations against the
+//    division's eleven;
+//  * 2 / (e^{2a} + 1): tanh_exp_abs_with, enumerated equal over its domain.
+// With wave_key below, soft cap + argmax of [256, 262144] at logits of standard
+// deviation 8 and cap 30: 135 -> 98 us (the soft cap alone 119 -> 92; at
+// deviation 1, where no value reaches the exponential, 91.8 -> 90.7).
+template <int N>
+__device__ __forceinline__ void softcap_lanes(float (&v)[N], const SoftCap& k) {
+    float hi = __builtin_fabsf(v[0]), lo = hi;
+#pragma unroll
+    for (int i = 1; i < N; ++i) {
+        hi = fmaxf(hi, __builtin_fabsf(v[i]));
+        lo = fminf(lo, __builtin_fabsf(v[i]));
+    }
+    float a[N], r[N];
+    if (k.plain && __builtin_amdgcn_ballot_w64(!(hi <= 0x1p60f && lo >= 0x1p-70f)) == 0) {
+        // NaN among plain values: max and min skip it, every step below
+        // propagates it and the range test leaves it to the series
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const float q0 = v[i] * k.rcp;
+            const float q1 = __builtin_fmaf(__builtin_fmaf(-q0, k.cap, v[i]), k.rcp, q0);
+            a[i] = __builtin_fabsf(__builtin_fmaf(__builtin_fmaf(-q1, k.cap, v[i]), k.rcp, q1));
+            r[i] = tanh_series_abs(a[i]);
+        }
+        // the quotient rounds monotonically: below 0.6249 cap none reaches 0.625
+        if (__builtin_amdgcn_ballot_w64(hi >= 0.6249f * k.cap) != 0) {
+#pragma unroll
+            for (int i = 0; i < N; ++i) {
+                const float big = tanh_exp_abs_with<DivPositive>(a[i]);
+                r[i] = a[i] >= 0.625f ? big : r[i];
+            }
+        }
+    } else {
+        bool need_exp = false;
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            a[i] = __builtin_fabsf(fdiv_rn(v[i], k.cap));
+            need_exp = need_exp || !tanh_series_range(a[i]);
+            r[i] = tanh_series_abs(a[i]);
+        }
+        if (__builtin_amdgcn_ballot_w64(need_exp) != 0) {
+#pragma unroll
+            for (int i = 0; i < N; ++i) {
+                const float big = tanh_exp_abs(a[i]);
+                r[i] = tanh_series_range(a[i]) ? r[i] : big;
+            }
+        }
+    }
+    // cap > 0: the quotient's sign is v's
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] = k.cap * __builtin_copysignf(r[i], v[i]);
+}
+
+// The wavefront's key over N float4 a lane, float4 u of lane l holding the
+// values from index first + (u * kLogitThreads + l) * 4 on: the wavefront's
+// maximum (NaN never raises it), then the last position that equals it, on the
+// scalar unit from the comparisons' lane masks -- two VALU operations a value
+// where folding a 64-bit key per value takes ten.  Wave-uniform.
+template <int N>
+__device__ __forceinline__ uint64_t wave_key(const float (&x)[4 * N], uint32_t first) {
+    float m = x[0];
+#pragma unroll
+    for (int i = 1; i < 4 * N; ++i) m = fmaxf(m, x[i]);
+    m = wave_max_tree_f32(m);
+    uint64_t key = 0;  // every value NaN
+    bool open = true;
+#pragma unroll
+    for (int u = N - 1; u >= 0; --u) {
+        uint64_t hit[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) hit[j] = __builtin_amdgcn_ballot_w64(x[4 * u + j] == m);
+        const uint64_t any = (hit[0] | hit[1]) | (hit[2] | hit[3]);
+        if (open && any != 0) {
+            open = false;
+            const uint32_t lane = 63u - static_cast<uint32_t>(__builtin_clzll(any));
+            const uint32_t j = (hit[3] >> lane) & 1 ? 3u : ((hit[2] >> lane) & 1 ? 2u : ((hit[1] >> lane) & 1 ? 1u : 0u));
+            key = argmax_key(m, first + (u * kLogitThreads + lane) * 4 + j);
+        }
+    }
+    return key;
+}
+
+// Reduce a workgroup's key (the wavefront's already when UNIFORM) and publish
+// it: the row's index when the row has one workgroup, otherwise the
+// workgroup's slot of the workspace.
+template <bool UNIFORM>
 __device__ __forceinline__ void publish_key(uint64_t key, uint32_t row, uint64_t* slots, uint32_t* selected) {
     __shared__ uint64_t wave_keys[kLogitThreads / kWave];
-    for (int off = kWave / 2; off > 0; off >>= 1) key = max_u64(key, __shfl_xor(key, off, kWave));
+    if (!UNIFORM)
+        for (int off = kWave / 2; off > 0; off >>= 1) key = max_u64(key, __shfl_xor(key, off, kWave));
     const uint32_t lane = threadIdx.x % kWave;
     const uint32_t wave = threadIdx.x / kWave;
     if (lane == 0) wave_keys[wave] = key;
@@ -101,8 +184,14 @@ __global__ __launch_bounds__(kLogitThreads) void argmax_finish_kernel(const uint
 
 // Rows of `count` logits; blockIdx.y = row, blockIdx.x = slice of
 // `per_block` values (a multiple of 1024 * U), walked in steps of 1024 * U.
-// Vector form: count % 4 == 0 and 16-byte aligned rows; every load of a
-// step is issued before its first value is processed.
+// 16-byte accesses at any 4-byte alignment (count >= 4; a count that is not a
+// multiple of 4 shifts every row); every load of a step is issued before its
+// first value is processed.  A float4 that runs past the row is loaded from
+// the row's last 4 values; the ones in front of its own position belong to
+// the thread before it and are neither stored nor counted.  [256, 50257] (one
+// value a thread before): 39.3 -> 24.8 us, argmax of [256, 32001] 16.5 -> 9.4.
+typedef f32x4 f32x4_row __attribute__((aligned(4)));
+
 template <bool CAP, bool ARG, int U>
 __global__ __launch_bounds__(kLogitThreads) void logits_vec_kernel(const float* in, float* out, uint32_t count,
                                                                    uint32_t per_block, float cap, uint64_t* slots,
@@ -111,34 +200,58 @@ __global__ __launch_bounds__(kLogitThreads) void logits_vec_kernel(const float* 
     const uint64_t base = static_cast<uint64_t>(row) * count;
     const uint32_t first = blockIdx.x * per_block;
     const uint32_t last = count - first < per_block ? count : first + per_block;
+    const SoftCap k = soft_cap(CAP ? cap : 1.0f);
+    const uint32_t wave = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(threadIdx.x / kWave));
     uint64_t key = 0;
     for (uint32_t begin = first; begin < last; begin += kLogitThreads * 4 * U) {
-        f32x4 v[U];
+        float x[4 * U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const uint32_t i = begin + (u * kLogitThreads + threadIdx.x) * 4;
-            const uint32_t ic = i < last ? i : last - 4;  // in-bounds duplicate for the idle tail
-            v[u] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(in + base + ic));
+            const uint32_t ic = min(i, count - 4);
+            const f32x4 v = __builtin_nontemporal_load(reinterpret_cast<const f32x4_row*>(in + base + ic));
+            x[4 * u] = v.x;
+            x[4 * u + 1] = v.y;
+            x[4 * u + 2] = v.z;
+            x[4 * u + 3] = v.w;
         }
+        if (CAP) softcap_lanes(x, k);
+        const bool whole = begin + kLogitThreads * 4 * U <= last;  // workgroup-uniform
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const uint32_t i = begin + (u * kLogitThreads + threadIdx.x) * 4;
-            float x[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
-            if (CAP) softcap_lanes(x, cap);
-            if (i < last) {
-                if (CAP && out)
-                    __builtin_nontemporal_store(f32x4{x[0], x[1], x[2], x[3]}, reinterpret_cast<f32x4*>(out + base + i));
-                if (ARG) {
+            if (CAP && out) {
+                if (whole || i + 4 <= last) {
+                    __builtin_nontemporal_store(f32x4{x[4 * u], x[4 * u + 1], x[4 * u + 2], x[4 * u + 3]},
+                                                reinterpret_cast<f32x4_row*>(out + base + i));
+                } else if (i < last) {
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) key = max_u64(key, argmax_key(x[j], i + j));
+                    for (int j = 0; j < 4; ++j)
+                        if (count - 4 + j >= i) out[base + count - 4 + j] = x[4 * u + j];
                 }
             }
+            if (ARG && !whole) {
+                // position j of this float4 is index i + j: shift the tail's
+                // values down and fill with NaN, which never wins
+                const uint32_t skip = i + 4 <= last ? 0u : (i < last ? i + 4 - last : 4u);
+                float y[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    y[j] = __builtin_nanf("");
+#pragma unroll
+                    for (int s = 0; s < 4; ++s)
+                        if (j + s < 4) y[j] = skip == static_cast<uint32_t>(s) ? x[4 * u + j + s] : y[j];
+                }
+#pragma unroll
+                for (int j = 0; j < 4; ++j) x[4 * u + j] = y[j];
+            }
         }
+        if (ARG) key = max_u64(key, wave_key<U>(x, begin + wave * (kWave * 4)));
     }
-    if (ARG) publish_key(key, row, slots, selected);
+    if (ARG) publish_key<true>(key, row, slots, selected);
 }
 
-// Any width or alignment: one value per thread per step.
+// Rows of fewer than 4 values: one value per thread per step.
 template <bool CAP, bool ARG>
 __global__ __launch_bounds__(kLogitThreads) void logits_scalar_kernel(const float* in, float* out, uint32_t count,
                                                                       uint32_t per_block, float cap, uint64_t* slots,
@@ -147,14 +260,15 @@ __global__ __launch_bounds__(kLogitThreads) void logits_scalar_kernel(const floa
     const uint64_t base = static_cast<uint64_t>(row) * count;
     const uint32_t begin = blockIdx.x * per_block;
     const uint32_t end = count - begin < per_block ? count : begin + per_block;
+    const SoftCap k = soft_cap(CAP ? cap : 1.0f);
     uint64_t key = 0;
     for (uint32_t i = begin + threadIdx.x; i < end; i += kLogitThreads) {
         float x[1] = {in[base + i]};
-        if (CAP) softcap_lanes(x, cap);
+        if (CAP) softcap_lanes(x, k);
         if (CAP && out) out[base + i] = x[0];
         if (ARG) key = max_u64(key, argmax_key(x[0], i));
     }
-    if (ARG) publish_key(key, row, slots, selected);
+    if (ARG) publish_key<false>(key, row, slots, selected);
 }
 
 // The grid of a soft cap / argmax over rows x count values: `blocks`
@@ -164,10 +278,9 @@ struct RowSplit {
     uint32_t blocks, per_block;
 };
 
-RowSplit row_split(const float* in, const float* out, uint32_t rows, uint32_t count) {
+RowSplit row_split(bool vec, uint32_t rows, uint32_t count) {
     RowSplit r;
-    r.vec = count % 4 == 0 && (reinterpret_cast<uintptr_t>(in) & 15) == 0 &&
-            (!out || (reinterpret_cast<uintptr_t>(out) & 15) == 0);
+    r.vec = vec;
     // large batches: steps of 4096 values; a single row: 1024, for more
     // workgroups in flight.  At most kArgmaxSlotsPerRow workgroups per row:
     // longer rows give each workgroup several steps.
@@ -182,6 +295,16 @@ RowSplit row_split(const float* in, const float* out, uint32_t rows, uint32_t co
     return r;
 }
 
+// The split that the no-allocation entry point's limit is stated in: rows
+// that are not a multiple of 4 values, or not 16-byte aligned, count their
+// workgroups in steps of 1024 values at any batch size.  The launch itself
+// needs at most as many.
+RowSplit limit_split(const float* in, const float* out, uint32_t rows, uint32_t count) {
+    return row_split(count % 4 == 0 && (reinterpret_cast<uintptr_t>(in) & 15) == 0 &&
+                         (!out || (reinterpret_cast<uintptr_t>(out) & 15) == 0),
+                     rows, count);
+}
+
 // Rows one launch can cover with `slot_count` workspace slots (a row split
 // over one workgroup writes its result directly and needs none).
 uint32_t row_launch_rows(uint32_t blocks, uint32_t slot_count) {
@@ -191,7 +314,7 @@ uint32_t row_launch_rows(uint32_t blocks, uint32_t slot_count) {
 template <bool CAP, bool ARG>
 hipError_t launch_rows(hipStream_t stream, const float* in, float* out, uint32_t* selected, uint32_t rows,
                        uint32_t count, float cap, uint64_t* slots, uint32_t slot_count) {
-    const RowSplit split = row_split(in, out, rows, count);
+    const RowSplit split = row_split(count >= 4, rows, count);
     const bool vec = split.vec, wide = split.wide;
     const uint32_t blocks = split.blocks, per_block = split.per_block;
     const uint32_t rows_per_launch = row_launch_rows(blocks, slot_count);
@@ -227,10 +350,11 @@ hipError_t launch_rows(hipStream_t stream, const float* in, float* out, uint32_t
 __global__ __launch_bounds__(kLogitThreads) void softcap_vec_kernel(const float* in, float* out, uint64_t n4,
                                                                     float cap) {
     const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
+    const SoftCap k = soft_cap(cap);
     for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n4; i += stride) {
         const f32x4 v = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(in) + i);
         float x[4] = {v.x, v.y, v.z, v.w};
-        softcap_lanes(x, cap);
+        softcap_lanes(x, k);
         __builtin_nontemporal_store(f32x4{x[0], x[1], x[2], x[3]}, reinterpret_cast<f32x4*>(out) + i);
     }
 }
@@ -238,9 +362,10 @@ __global__ __launch_bounds__(kLogitThreads) void softcap_vec_kernel(const float*
 __global__ __launch_bounds__(kLogitThreads) void softcap_scalar_kernel(const float* in, float* out, uint64_t begin,
                                                                        uint64_t n, float cap) {
     const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
+    const SoftCap k = soft_cap(cap);
     for (uint64_t i = begin + static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += stride) {
         float x[1] = {in[i]};
-        softcap_lanes(x, cap);
+        softcap_lanes(x, k);
         out[i] = x[0];
     }
 }
@@ -267,13 +392,13 @@ hipError_t launch_logits_f32(hipStream_t stream, const float* logits, float* cap
 
 uint32_t logits_launches(const float* logits, const float* capped, uint32_t rows, uint32_t count,
                          uint32_t slot_count) {
-    const RowSplit split = row_split(logits, capped, rows, count);
+    const RowSplit split = limit_split(logits, capped, rows, count);
     const uint32_t per = row_launch_rows(split.blocks, slot_count);
     return per == 0 ? 0u : (rows + per - 1) / per;
 }
 
 uint32_t logits_row_blocks(const float* logits, const float* capped, uint32_t rows, uint32_t count) {
-    return row_split(logits, capped, rows, count).blocks;
+    return limit_split(logits, capped, rows, count).blocks;
 }
 
 // ---------------------------------------------------------------------------

@@ -1,0 +1,70 @@
+"""The soft cap + argmax rows that are not a multiple of 4 values or not
+16-byte aligned (16-byte accesses at 4-byte alignment), their tails, in place,
+and the soft cap's shorter divisions over caps and magnitudes at the edges of
+the range that takes them."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+f32 = np.float32
+
+
+def _rows(seed, rows, count, std):
+    r = np.random.default_rng(seed)
+    x = (r.standard_normal(rows * count) * std).astype(f32).reshape(rows, count)
+    for i in range(rows):  # ties on the maximum, the last one at or near the row's end
+        x[i, [i % count, max(0, count - 1 - i % 6)]] = f32(9 * std)
+        if count > 8:
+            x[i, (7 * i + 3) % count] = np.nan
+    return x.reshape(-1)
+
+
+def _same(got, exp):
+    return np.array_equal(np.where(np.isnan(got), 0, got).view(np.uint32), np.where(np.isnan(exp), 0, exp).view(np.uint32)) \
+        and np.array_equal(np.isnan(got), np.isnan(exp))
+
+
+@pytest.mark.parametrize("rows,count", [(1, 3), (5, 4), (7, 5), (9, 7), (3, 1023), (3, 1026), (2, 4095), (2, 4099),
+                                        (1, 32001), (130, 32001), (85, 50257), (3, 1400005)])
+@pytest.mark.parametrize("offset,in_place", [(0, False), (4, False), (12, True)])
+def test_rows(rt, ora, rows, count, offset, in_place):
+    x = _rows(rows + count, rows, count, 8.0)
+    exp_c, exp_s = ora.softcap_argmax_rows(x, rows, count, 30.0)
+    src = rt.empty(x.size + 8).offset(offset)
+    src.upload(x)
+    dst = src if in_place else rt.empty(x.size + 8).offset(offset)
+    sel = rt.empty(rows, np.uint32)
+    rt.softcap_argmax(src, dst, sel, rows, count, 30.0)
+    rt.sync()
+    assert _same(dst.download(x.size), exp_c)
+    assert np.array_equal(sel.download(rows, np.uint32), exp_s)
+    src.upload(x)
+    rt.argmax(src, sel, rows, count)
+    rt.sync()
+    assert np.array_equal(sel.download(rows, np.uint32), ora.softcap_argmax_rows(x, rows, count, 0.0)[1])
+    for b in {id(src): src, id(dst): dst}.values():
+        b.ptr -= offset
+        rt.free(next(o for o in rt._buffers if o.ptr == b.ptr))
+
+
+# 0x3fffffff has an all-ones significand; 2^-20 and 2^20 bound the plain caps
+CAPS = [30.0, 50.0, 1.0, 0.37, float(np.array([0x3FFFFFFF], np.uint32).view(f32)[0]), 3.0, 7.0e5, 2.0 ** -20, 2.0 ** 20,
+        2.0 ** -21, 1.5e6, 1e-30, 1e30]
+
+
+@pytest.mark.parametrize("cap", CAPS)
+def test_caps_and_magnitudes(rt, ora, cap):
+    r = np.random.default_rng(5)
+    mant = (1.0 + r.random((400, 1024))).astype(f32)
+    sign = np.where(r.random(mant.shape) < 0.5, -1, 1).astype(f32)
+    near = np.ldexp(mant, r.integers(-3, 4, mant.shape)).astype(f32) * f32(cap)  # about the cap: both tanh ranges
+    far = np.ldexp(mant, r.integers(-75, 66, mant.shape)).astype(f32)            # across the plain range's edges
+    edge = np.tile(np.array([2.0 ** -70, 2.0 ** 60, 1.0], f32), 342)[:1024] * mant[:8]
+    with np.errstate(over="ignore"):
+        x = np.concatenate([near * sign, far * sign, edge, -edge]).astype(f32).reshape(-1)
+    buf, out = rt.upload(x), rt.empty(x.size)
+    rt.softcap(buf, out, x.size, cap)
+    rt.sync()
+    assert _same(out.download(x.size), ora.softcap(x, cap))
+    rt.free(buf)
+    rt.free(out)
