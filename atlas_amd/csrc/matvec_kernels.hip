@@ -19,18 +19,25 @@
 // matvec_rms_fused_parity.rs: max-abs < 1e-3); the summation order here is
 // this kernel's own, deterministic run to run.
 //
-// Layout on CDNA: the op streams the weight matrix once (it is HBM-bound;
-// MFMA does not apply to one token).  One wavefront owns a tile of 16
-// consecutive output rows -- a contiguous byte range of the weight matrix --
-// and stages it into LDS with 128-bit loads, all issued before the first
-// wait.  Meanwhile the lanes form y = x * w (the normalised input before its
-// scalar) in LDS with the per-block sums of y and the row sum of squares.
-// Lane (g, s), g < 64/LPR, s < LPR, then keeps the y values of blocks
-// s, s + LPR, ... in registers and applies them to rows g, g + 64/LPR, ...
-// of the tile: 16 nibbles per byte pair decoded with masks and
-// v_cvt_f32_ubyte, sum_j q_j * y_j accumulated in f32, and the Q4_0 offset
-// folded as d * (acc - 8 * sum(y)).  The LPR partial sums of a row are
-// reduced with cross-lane shuffles inside the row's lane group.
+// Layout on CDNA: the op streams the weight matrix once, and a vector dot of
+// 4-bit codes costs more VALU work (a conversion and an FMA per weight) than
+// its bytes take to arrive, so the codes meet the input on the matrix cores as
+// integers (v_mfma_i32_4x4x4_16b_i8: 16 independent 4 x 4 x 4 products):
+//  * each 32-value block of y = x * w becomes 31-bit fixed point under the
+//    block's largest |y| (relative 2^-31; f32 itself holds 2^-24) and is split
+//    into four signed byte digits; the digits of four consecutive values are
+//    one word per digit, the A operand's four rows;
+//  * a lane holds one weight row's block as loaded, 16 (q - 8) in the bytes of
+//    eight words by a mask and a shift (q ^ 8 in a byte's high nibble is
+//    16 (q - 8) in two's complement), the B operand's columns: lane l is row
+//    l % 4 of the wavefront's four and block l / 4 of the pass's sixteen;
+//  * eight products accumulate a block exactly in i32, one register per digit
+//    and in the lane of its row; the digits meet in two 24-bit halves, one f32
+//    fma, and the block's scale d goes on with the row's running sum.
+// ~45 VALU operations a block instead of ~85, 32 bytes of the input read from
+// LDS per lane and block instead of 128, and a dot whose only roundings are
+// three per block: the error against float64 falls from 3e-8 to 9e-9 of the
+// sum of magnitudes.
 #include "device_common.hpp"
 #include "launch.hpp"
 
@@ -38,142 +45,139 @@ namespace atlas {
 namespace {
 
 constexpr uint32_t kQ4Block = 18;  // bytes per 32 values
+constexpr uint32_t kPassBlocks = 16, kPassRows = 4;
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef u32x4 u32x4_block __attribute__((aligned(2)));  // a block's codes start 2 bytes into its 18
 
-// Stage `bytes` (even) starting at `src` into LDS: 16-byte loads when the
-// source is 16-byte aligned (the tail in 2-byte units), else 2-byte loads.
-// A pass issues K loads per lane before the first LDS write (K = 4 covers a
-// wavefront's 4 rows of 864 bytes, the Gemma hidden width, in one pass).  Load and store
-// indices are both clamped to the last unit (lanes past the end copy that
-// unit again, writing the value it already holds), so no access is
-// conditional and the compiler cannot sink a load into a guarded store and
-// serialise the pass.
-template <int K, typename U>
-__device__ __forceinline__ void stage_units(uint8_t* dst, const uint8_t* src, uint32_t units, uint32_t lane) {
-    for (uint32_t base = 0; base < units; base += K * kWave) {
-        U v[K];
-#pragma unroll
-        for (int k = 0; k < K; ++k) v[k] = reinterpret_cast<const U*>(src)[min(base + lane + k * kWave, units - 1)];
-#pragma unroll
-        for (int k = 0; k < K; ++k) reinterpret_cast<U*>(dst)[min(base + lane + k * kWave, units - 1)] = v[k];
-    }
+template <int CTRL>
+__device__ __forceinline__ uint32_t dpp_u32(uint32_t v) {
+    return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), CTRL, 0xf, 0xf, false));
 }
-
-__device__ __forceinline__ void stage_tile(uint8_t* dst, const uint8_t* src, uint32_t bytes, uint32_t lane) {
-    uint32_t done = 0;
-    if ((reinterpret_cast<uintptr_t>(src) & 15) == 0) {
-        const uint32_t n16 = bytes / 16;
-        if (n16) stage_units<4, uint4>(dst, src, n16, lane);
-        done = n16 * 16;
-    }
-    if (bytes > done) stage_units<8, uint16_t>(dst + done, src + done, (bytes - done) / 2, lane);
-}
-
-// Sum over aligned groups of LPR lanes; every lane of a group gets the total.
-// Inside a 16-lane DPP row the butterfly is quad_perm (xor 1, xor 2),
-// row_half_mirror and row_mirror (VALU ops, no LDS); wider groups add
-// cross-row shuffles.
 template <int CTRL>
 __device__ __forceinline__ float dpp_f32(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
+    return __uint_as_float(dpp_u32<CTRL>(__float_as_uint(v)));
 }
 
-template <int LPR>
-__device__ __forceinline__ float group_sum(float v) {
-    v += dpp_f32<0xb1>(v);                 // quad_perm [1,0,3,2]
-    v += dpp_f32<0x4e>(v);                 // quad_perm [2,3,0,1]
-    if (LPR >= 8) v += dpp_f32<0x141>(v);   // row_half_mirror
-    if (LPR >= 16) v += dpp_f32<0x140>(v);  // row_mirror
-    if (LPR >= 32) v += __shfl_xor(v, 16, kWave);
-    if (LPR >= 64) v += __shfl_xor(v, 32, kWave);
-    return v;
+// Largest value over aligned groups of 8 lanes.
+__device__ __forceinline__ uint32_t group8_max(uint32_t v) {
+    v = max(v, dpp_u32<0xb1>(v));         // quad_perm [1,0,3,2]
+    v = max(v, dpp_u32<0x4e>(v));         // quad_perm [2,3,0,1]
+    return max(v, dpp_u32<0x141>(v));     // row_half_mirror
 }
 
-// The Q4_0 block at LDS byte offset `off` (even): its f16 scale d and its
-// 16 quant bytes as four dwords, read with 4-byte LDS loads.  An offset that
-// is 0 mod 4 holds the scale in the low half of the first dword (the five
-// dwords end 2 bytes past the block, still inside the LDS allocation); an
-// offset that is 2 mod 4 holds it in the high half of the dword before the
-// quant bytes, which are then dword aligned.
-__device__ __forceinline__ void load_q4_block(const uint8_t* lds, uint32_t off, float& d, uint32_t (&q)[4]) {
-    if ((off & 3) == 0) {
-        const uint32_t* p = reinterpret_cast<const uint32_t*>(lds + off);
-        const uint32_t w0 = p[0], w1 = p[1], w2 = p[2], w3 = p[3], w4 = p[4];
-        d = h2f(static_cast<uint16_t>(w0));
-        q[0] = __builtin_amdgcn_alignbit(w1, w0, 16);
-        q[1] = __builtin_amdgcn_alignbit(w2, w1, 16);
-        q[2] = __builtin_amdgcn_alignbit(w3, w2, 16);
-        q[3] = __builtin_amdgcn_alignbit(w4, w3, 16);
-    } else {
-        const uint32_t* p = reinterpret_cast<const uint32_t*>(lds + off - 2);
-        d = h2f(static_cast<uint16_t>(p[0] >> 16));
-        q[0] = p[1];
-        q[1] = p[2];
-        q[2] = p[3];
-        q[3] = p[4];
-    }
+// Sum over the lanes with the same lane % 4; every lane gets its total.
+__device__ __forceinline__ float sum_of_row(float v) {
+    v += dpp_f32<0x124>(v);  // row_ror:4
+    v += dpp_f32<0x128>(v);  // row_ror:8
+    v += __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), 0x401f));  // xor 16
+    return v + __shfl_xor(v, 32, kWave);
 }
 
-// sum_j q_j * y_j over one Q4_0 block's 32 values (nibble codes 0..15):
-// byte j of q holds codes j (low nibble) and j + 16 (high nibble).
-__device__ __forceinline__ float q4_block_dot(const uint32_t (&q)[4], const float (&y)[32]) {
-    float acc = 0.0f;
+// Four values as signed byte digits: word p holds digit p (weight 256^p) of
+// the four, after scaling by 2^shift (|v 2^shift| <= 2^30).
+__device__ __forceinline__ void digit_words(const f32x4 v, int shift, uint32_t (&word)[4]) {
+    uint32_t t[4];
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
-        uint32_t lo = q[w] & 0x0f0f0f0fu, hi = (q[w] >> 4) & 0x0f0f0f0fu;
-        // hide the masks' known-zero bits: knowing them, the compiler extracts
-        // each nibble with a bitfield extract before a byte-0 conversion
-        // (two instructions) instead of converting byte k directly (one)
-        __asm__("" : "+v"(lo), "+v"(hi));
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {  // byte-wise conversions (v_cvt_f32_ubyte0..3)
-            acc = __builtin_fmaf(static_cast<float>((lo >> (8 * k)) & 0xffu), y[4 * w + k], acc);
-            acc = __builtin_fmaf(static_cast<float>((hi >> (8 * k)) & 0xffu), y[4 * w + k + 16], acc);
-        }
+    for (int i = 0; i < 4; ++i) {
+        const int q = static_cast<int>(__builtin_ldexpf(v[i], shift));
+        // a digit d in [-128, 127] is the byte d + 128 of q + 0x808080 (the
+        // top one has no bias), so clearing the bias leaves two's complement
+        t[i] = (static_cast<uint32_t>(q) + 0x00808080u) ^ 0x00808080u;
     }
-    return acc;
+    // 4 x 4 byte transpose
+    const uint32_t a = __builtin_amdgcn_perm(t[1], t[0], 0x05010400u), b = __builtin_amdgcn_perm(t[1], t[0], 0x07030602u);
+    const uint32_t c = __builtin_amdgcn_perm(t[3], t[2], 0x05010400u), d = __builtin_amdgcn_perm(t[3], t[2], 0x07030602u);
+    word[0] = __builtin_amdgcn_perm(c, a, 0x05040100u);
+    word[1] = __builtin_amdgcn_perm(c, a, 0x07060302u);
+    word[2] = __builtin_amdgcn_perm(d, b, 0x05040100u);
+    word[3] = __builtin_amdgcn_perm(d, b, 0x07060302u);
+}
+
+// A block's 18 bytes behind five dwords at `p`, the 4-byte boundary at or
+// below it: `high` says that it starts at the second half of the first.  The
+// f16 scale comes first, the codes follow (the dwords end at most 2 bytes past
+// the block: the LDS has 4 spare).
+__device__ __forceinline__ void read_block(const uint32_t* p, bool high, float& d, uint32_t (&q)[4]) {
+    const uint32_t w[5] = {p[0], p[1], p[2], p[3], p[4]};
+    const uint32_t sel = high ? 0x07060504u : 0x05040302u;
+    d = h2f(static_cast<uint16_t>(w[0] >> (high ? 16 : 0)));
+#pragma unroll
+    for (int i = 0; i < 4; ++i) q[i] = __builtin_amdgcn_perm(w[i + 1], w[i], sel);
 }
 
 constexpr uint32_t kWaves = 4;  // wavefronts per workgroup
-// y is stored block by block with a 36-float stride: the 16 or 32 lanes of
-// a row group read 16-byte pieces of consecutive blocks, and a 144-byte
-// stride puts those pieces on distinct LDS banks (a 128-byte stride would
-// put them all on the same four).
-constexpr uint32_t kYStride = 36;
 
-// LPR lanes per output row (one row per lane group), NBT blocks per lane
-// (blocks per row <= LPR * NBT).  A workgroup owns kWaves * 64 / LPR rows.
-template <int LPR, int NBT, bool ONEPASS>
-__global__ __launch_bounds__(256) void q4_0_matvec_kernel(MatvecArgs a) {
-    constexpr uint32_t kGroups = kWave / LPR;           // rows per wavefront
-    constexpr uint32_t kRows = kWaves * kGroups;        // rows per workgroup
-    constexpr int kJ = (LPR * NBT * 32 / 4 + 255) / 256;  // float4 of x per thread
+// LDS bytes of the input's digits and exponents, and of a wavefront's region
+// for one group's rows (NBT passes of 4 x 16 blocks, 4 bytes over-read).
+__host__ __device__ constexpr uint32_t plane_bytes(uint32_t nb) { return (nb * 132 + 15) & ~15u; }
+__host__ __device__ constexpr uint32_t stage_bytes(int nbt) { return 4 * 16 * 18 * nbt + 16; }
+
+// NBT passes of 16 blocks per wavefront and group of four rows.
+// STAGED: a wavefront takes `groups` groups of four consecutive rows, each
+// group's one contiguous span loaded with coalesced 16-byte loads and staged
+// in the wavefront's LDS region while the group before it is computed.
+// Otherwise (one group) the lanes load their blocks themselves: no LDS round
+// trip before the dot, but 16-byte accesses 18 bytes apart, which the address
+// unit takes ~225 cycles a pass over; KS wavefronts share a group's rows, NBT
+// passes each.
+template <int NBT, int KS, bool STAGED>
+__global__ __launch_bounds__(256) void q4_0_matvec_kernel(MatvecArgs a, uint32_t groups) {
+    static_assert(!STAGED || KS == 1, "a staged row belongs to one wavefront");
+    constexpr int kJ = (NBT * KS * kPassBlocks * 32 / 4 + 255) / 256;  // float4 of x per thread
+    constexpr int kLoads = STAGED ? (4 * 18 * NBT + 63) / 64 : NBT;  // 16-byte loads per lane and group
     extern __shared__ __align__(16) uint8_t smem[];
-    const uint32_t tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
-    const uint32_t g = lane / LPR, s = lane % LPR;
+    __shared__ float ss_part[kWaves], bad_part[kWaves], red[KS > 1 ? kWaves * kPassRows : 1];
+    const uint32_t tid = threadIdx.x, lane = tid % kWave;
+    const uint32_t wave = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(tid / kWave));
     const uint32_t n = a.input_width, n4 = n / 4, nb = n / 32, row_bytes = nb * kQ4Block;
+    const uint32_t rows = kPassRows * groups * kWaves / KS;  // rows per workgroup
 
     // The projection this workgroup's rows belong to (segments are tile ranges).
-    const uint32_t t = blockIdx.x;
-    const uint32_t si = (a.segments > 2 && t >= a.tile_begin[2]) ? 2 : ((a.segments > 1 && t >= a.tile_begin[1]) ? 1 : 0);
+    const uint32_t tile = blockIdx.x;
+    const uint32_t si = (a.segments > 2 && tile >= a.tile_begin[2]) ? 2 : ((a.segments > 1 && tile >= a.tile_begin[1]) ? 1 : 0);
     const uint8_t* weights = si == 0 ? a.weights[0] : (si == 1 ? a.weights[1] : a.weights[2]);
     float* out = si == 0 ? a.output[0] : (si == 1 ? a.output[1] : a.output[2]);
     const uint32_t width = si == 0 ? a.width[0] : (si == 1 ? a.width[1] : a.width[2]);
     const uint32_t begin = si == 0 ? a.tile_begin[0] : (si == 1 ? a.tile_begin[1] : a.tile_begin[2]);
-    const uint32_t row0 = (t - begin) * kRows;
-    const uint32_t nrows = min(kRows, width - row0);
-    // this wavefront's rows: [wrow0, wrow0 + wrows) of the tile
-    const uint32_t wrow0 = min(wave * kGroups, nrows);
-    const uint32_t wrows = min(kGroups, nrows - wrow0);
+    const uint32_t part = KS == 1 ? 0u : wave % KS;
+    const uint32_t row0 = (tile - begin) * rows + (wave / KS) * (kPassRows * groups);  // the wavefront's first row
+    const uint32_t g = lane % kPassRows, s = lane / kPassRows;
+    const uint32_t b0 = KS == 1 ? 0u : min(part * (NBT * kPassBlocks), nb - 1);  // its first block of each row
+    const uint32_t cnt = min(nb - b0, NBT * kPassBlocks);
 
-    uint8_t* tile = smem;                                                         // kRows * row_bytes
-    float* ys = reinterpret_cast<float*>(smem + ((kRows * row_bytes + 15) & ~15u));  // nb * kYStride floats
-    float* block_sums = ys + nb * kYStride;                                       // nb floats
-    float* partial = block_sums + nb;                                             // kWaves floats
+    u32x4* planes = reinterpret_cast<u32x4*>(smem);                          // nb blocks x 4 digits x 8 words
+    int* block_exp = reinterpret_cast<int*>(smem + nb * 128);                // nb exponents
+    uint8_t* region = smem + plane_bytes(nb) + wave * stage_bytes(NBT);
 
-    // 1. input and RMS weight: every load of the workgroup issued up front
-    //    (indices clamped, duplicates not stored)
+    u32x4 q[kLoads];
+    uint16_t qd[STAGED ? 1 : NBT];
+    // rows past the end reload the last one
+    auto load_group = [&](uint32_t r) {
+        const uint32_t first = min(row0 + kPassRows * r, width - 1);
+        if constexpr (STAGED) {
+            // the last 16 bytes of a span overlap the ones before them
+            const uint8_t* span = weights + static_cast<size_t>(first) * row_bytes;
+            const uint32_t bytes = min(kPassRows, width - first) * row_bytes;
+#pragma unroll
+            for (int k = 0; k < kLoads; ++k)
+                q[k] = __builtin_nontemporal_load(
+                    reinterpret_cast<const u32x4_block*>(span + min(16u * (lane + 64u * k), bytes - 16u)));
+        } else {
+            const uint8_t* row = weights + static_cast<size_t>(min(first + g, width - 1)) * row_bytes;
+#pragma unroll
+            for (int t = 0; t < NBT; ++t) {
+                const uint8_t* blk = row + (b0 + min(s + kPassBlocks * t, cnt - 1)) * kQ4Block;
+                qd[t] = __builtin_nontemporal_load(reinterpret_cast<const uint16_t*>(blk));
+                q[t] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_block*>(blk + 2));
+            }
+        }
+    };
+
+    // 1. input and RMS weight, then the first group's weights (the dominant
+    //    stream): every load issued up front, indices clamped
     const bool rms = a.rms_weight != nullptr;
     f32x4 xv[kJ], wv[kJ];
 #pragma unroll
@@ -182,127 +186,153 @@ __global__ __launch_bounds__(256) void q4_0_matvec_kernel(MatvecArgs a) {
         xv[j] = reinterpret_cast<const f32x4*>(a.input)[c];
         wv[j] = rms ? reinterpret_cast<const f32x4*>(a.rms_weight)[c] : f32x4{1.0f, 1.0f, 1.0f, 1.0f};
     }
+    load_group(0);
 
-    // 2. this wavefront's weight rows (the dominant stream), staged into LDS.
-    //    ONEPASS (16-byte aligned rows of a 16-byte multiple, at most 4 KiB
-    //    per wavefront -- four 864-byte rows): the loads land in registers
-    //    and are written to LDS only after step 3, so y = x * w and the sums
-    //    overlap the HBM round trip.  Loads and stores are unconditional, with
-    //    clamped indices: a branch around either lets the compiler merge the
-    //    registers or sink the loads to the stores, which waits for the data
-    //    before step 3.  A wavefront without rows (the tail of the last tile)
-    //    copies its tile's first row into the unused slot at row nrows.
-    const uint8_t* wsrc = weights + static_cast<size_t>(row0 + (wrows ? wrow0 : 0u)) * row_bytes;
-    const uint32_t n16 = (wrows ? wrows : 1u) * row_bytes / 16;
-    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-    u32x4 w0, w1, w2, w3;
-    if constexpr (ONEPASS) {
-        const u32x4* src = reinterpret_cast<const u32x4*>(wsrc);  // read once: nontemporal
-        w0 = __builtin_nontemporal_load(src + min(lane, n16 - 1));
-        w1 = __builtin_nontemporal_load(src + min(lane + kWave, n16 - 1));
-        w2 = __builtin_nontemporal_load(src + min(lane + 2 * kWave, n16 - 1));
-        w3 = __builtin_nontemporal_load(src + min(lane + 3 * kWave, n16 - 1));
-    } else {
-        if (wrows) stage_tile(tile + wrow0 * row_bytes, wsrc, wrows * row_bytes, lane);
-    }
-
-    // 3. y = x * w (or x), the per-block sums of y (a block is 8 float4, held
-    //    by 8 consecutive threads) and the sum of squares
+    // 2. y = x * w (or x) as digits, and the sum of squares; a block is 8
+    //    float4, held by 8 consecutive threads
     float ss = 0.0f;
+    bool bad = false;
 #pragma unroll
     for (int j = 0; j < kJ; ++j) {
         const uint32_t c = min(tid + 256u * j, n4 - 1);  // duplicates recompute the last float4
         const f32x4 x = xv[j], w = wv[j];
         f32x4 y = x;
         if (rms) y = f32x4{x.x * w.x, x.y * w.y, x.z * w.z, x.w * w.w};
-        const float bsum = group_sum<8>((y.x + y.y) + (y.z + y.w));
+        uint32_t m = 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) m = max(m, __float_as_uint(y[i]) & 0x7fffffffu);
+        const int e = static_cast<int>(group8_max(m) >> 23);  // |y| < 2^(e - 126) over the block
+        bad = bad || e == 255;
+        uint32_t word[4];
+        digit_words(y, 156 - e, word);
         if (tid + 256u * j < n4) {
             if (rms) ss = ss + x.x * x.x + x.y * x.y + x.z * x.z + x.w * x.w;
-            *reinterpret_cast<f32x4*>(ys + (c / 8) * kYStride + 4 * (c % 8)) = y;
-            if (c % 8 == 0) block_sums[c / 8] = bsum;
+            uint32_t* dst = reinterpret_cast<uint32_t*>(planes) + (c / 8) * 32 + c % 8;
+#pragma unroll
+            for (int p = 0; p < 4; ++p) dst[8 * p] = word[p];
+            if (c % 8 == 0) block_exp[c / 8] = e - 160;  // the codes carry a factor 16
         }
     }
-    ss = group_sum<kWave>(ss);
-    if (lane == 0) partial[wave] = ss;
-    // y, the block sums and the partial sums are shared; the weight rows are
-    // the wavefront's own, so it waits for its rows alone and starts its dot
-    // while the workgroup's other rows may still be in flight (gate/up at
-    // one token: 5.30 against 5.39 us with the rows written before the
-    // barrier)
-    __syncthreads();
-    if constexpr (ONEPASS) {
-        u32x4* dst = reinterpret_cast<u32x4*>(tile + wrow0 * row_bytes);
-        dst[min(lane, n16 - 1)] = w0;
-        dst[min(lane + kWave, n16 - 1)] = w1;
-        dst[min(lane + 2 * kWave, n16 - 1)] = w2;
-        dst[min(lane + 3 * kWave, n16 - 1)] = w3;
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    ss = wave_sum_tree_f32(ss);
+    const bool any_bad = __builtin_amdgcn_ballot_w64(bad) != 0;
+    if (lane == 0) {
+        ss_part[wave] = ss;
+        bad_part[wave] = any_bad ? __builtin_nanf("") : 0.0f;
     }
-    // The projection is held to a tolerance (this kernel's own summation
-    // order), so the inverse RMS takes the hardware reciprocal and reciprocal
-    // square root (each within 1 ulp): rsq(sum * rcp(n) + eps), a few ulp,
-    // where the IEEE form (two divisions and a square root) costs ~45
-    // instructions per wavefront.
-    float inv = 1.0f;
-    if (rms)
-        inv = __builtin_amdgcn_rsqf(((partial[0] + partial[1]) + (partial[2] + partial[3])) *
-                                        __builtin_amdgcn_rcpf(static_cast<float>(n)) + a.epsilon);
+    // y and the sums are shared; the weight rows are the wavefront's own
+    __syncthreads();
 
-    // 4. lane (g, s): row wrow0 + g, blocks s + LPR * i
-    const uint32_t row = wrow0 + g;
-    float acc = 0.0f;
-    if (g < wrows) {
-        const uint32_t row_off = row * row_bytes;
+    // The projection is held to a tolerance, so the inverse RMS takes the
+    // hardware reciprocal and reciprocal square root (each within 1 ulp):
+    // rsq(sum * rcp(n) + eps), a few ulp, where the IEEE form (two divisions
+    // and a square root) costs ~45 instructions per wavefront.
+    float nan = bad_part[0], sum = ss_part[0];  // NaN with an infinity or NaN in y
 #pragma unroll
-        for (int i = 0; i < NBT; ++i) {
-            const uint32_t b = s + LPR * i;
-            if (b < nb) {
-                float y[32];
+    for (int i = 1; i < kWaves; ++i) {
+        nan = nan + bad_part[i];
+        sum = sum + ss_part[i];
+    }
+    float inv = 1.0f;
+    if (rms) inv = __builtin_amdgcn_rsqf(sum * __builtin_amdgcn_rcpf(static_cast<float>(n)) + a.epsilon);
+
+    // 3. lane (g, s): row g of each group, blocks b0 + s + 16 pass
+    for (uint32_t r = 0; r < groups; ++r) {
+        if constexpr (STAGED) {
+            const uint32_t first = min(row0 + kPassRows * r, width - 1);
+            const uint32_t bytes = min(kPassRows, width - first) * row_bytes;
 #pragma unroll
-                for (int k = 0; k < 8; ++k) {
-                    const f32x4 v = *reinterpret_cast<const f32x4*>(ys + kYStride * b + 4 * k);
-                    y[4 * k] = v.x;
-                    y[4 * k + 1] = v.y;
-                    y[4 * k + 2] = v.z;
-                    y[4 * k + 3] = v.w;
-                }
-                float d;
-                uint32_t q[4];
-                load_q4_block(tile, row_off + b * kQ4Block, d, q);
-                acc = __builtin_fmaf(d, q4_block_dot(q, y) - 8.0f * block_sums[b], acc);
+            for (int k = 0; k < kLoads; ++k)
+                if (16u * (lane + 64u * k) < bytes)
+                    *reinterpret_cast<u32x4_block*>(region + min(16u * (lane + 64u * k), bytes - 16u)) = q[k];
+            if (r + 1 < groups) load_group(r + 1);
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        }
+        // Straight-line over the passes, so their product chains overlap.  A
+        // staged row's NBT passes end within 16 blocks of it: only the last
+        // pass has lanes past it, which read whatever the LDS holds there
+        // (inside the allocation) and are dropped; 16 blocks are 288 bytes, so
+        // a lane's half-word parity is the same in every pass.  An unstaged
+        // share may be shorter: its lanes repeat the last block.
+        float d[NBT];
+        int e[NBT];
+        i32x4 p[NBT];
+#pragma unroll
+        for (int t = 0; t < NBT; ++t) {
+            const uint32_t at = STAGED ? s + kPassBlocks * t : b0 + min(s + kPassBlocks * t, cnt - 1);
+            const i32x4* src = reinterpret_cast<const i32x4*>(planes) + at * 8 + g * 2;
+            const i32x4 y0 = src[0], y1 = src[1];
+            e[t] = block_exp[at];
+            uint32_t c[4];
+            if constexpr (STAGED) {
+                const uint32_t off = g * row_bytes + s * kQ4Block;
+                read_block(reinterpret_cast<const uint32_t*>(region + (off & ~3u)) + t * (kPassBlocks * kQ4Block / 4),
+                           (off & 2u) != 0, d[t], c);
+            } else {
+                d[t] = h2f(qd[t]);
+#pragma unroll
+                for (int w = 0; w < 4; ++w) c[w] = q[t][w];
+            }
+            p[t] = i32x4{0, 0, 0, 0};
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                const uint32_t lo = ((c[w] << 4) ^ 0x80808080u) & 0xf0f0f0f0u, hi = (c[w] ^ 0x80808080u) & 0xf0f0f0f0u;
+                p[t] = __builtin_amdgcn_mfma_i32_4x4x4i8(y0[w], static_cast<int>(lo), p[t], 0, 0, 0);
+                p[t] = __builtin_amdgcn_mfma_i32_4x4x4i8(y1[w], static_cast<int>(hi), p[t], 0, 0, 0);
             }
         }
-    }
-    const float total = group_sum<LPR>(acc);
-    if (s == 0 && g < wrows) {
-        if (a.ple)  // PLE input gate: GELU of the projection times the layer's PLE slice
-            out[row0 + row] = gelu_tanh_f32(total) * a.ple[a.ple_offset + row0 + row];
-        else
-            out[row0 + row] = rms ? total * inv : total;
+        float acc = 0.0f;
+#pragma unroll
+        for (int t = 0; t < NBT; ++t) {
+            const float lo = static_cast<float>(p[t].x + (p[t].y << 8)), hi = static_cast<float>(p[t].z + (p[t].w << 8));
+            const float sum = __builtin_fmaf(__builtin_ldexpf(__builtin_fmaf(hi, 65536.0f, lo), e[t]), d[t], acc);
+            const bool in = (STAGED && t < NBT - 1) || part * (NBT * kPassBlocks) + s + kPassBlocks * t < nb;
+            acc = in ? sum : acc;
+        }
+        if (STAGED) __builtin_amdgcn_wave_barrier();  // the region is read before the next group's stores
+        float total = sum_of_row(acc);
+        if constexpr (KS > 1) {
+            if (lane < kPassRows) red[wave * kPassRows + lane] = total;
+            __syncthreads();
+            if (part != 0) return;
+            total = 0.0f;
+#pragma unroll
+            for (int i = 0; i < KS; ++i) total = total + red[(wave + i) * kPassRows + g];
+        }
+        const uint32_t row = row0 + kPassRows * r + lane;
+        if (lane < kPassRows && row < width) {
+            const float v = total + nan;
+            if (a.ple)  // PLE input gate: GELU of the projection times the layer's PLE slice
+                out[row] = gelu_tanh_f32(v) * a.ple[a.ple_offset + row];
+            else
+                out[row] = rms ? v * inv : v;
+        }
     }
 }
 
-template <int LPR, int NBT>
-hipError_t launch_lpr(hipStream_t stream, MatvecArgs a) {
-    constexpr uint32_t kGroupsL = kWave / LPR;
-    constexpr uint32_t kRows = kWaves * (kWave / LPR);
+template <int NBT, int KS, bool STAGED>
+hipError_t launch_shape(hipStream_t stream, MatvecArgs a, uint32_t groups) {
+    const uint32_t rows = kPassRows * groups * kWaves / KS;
     uint32_t tiles = 0;
     for (uint32_t i = 0; i < a.segments; ++i) {
         a.tile_begin[i] = tiles;
-        tiles += (a.width[i] + kRows - 1) / kRows;
+        tiles += (a.width[i] + rows - 1) / rows;
     }
-    const uint32_t nb = a.input_width / 32;
-    const size_t lds = ((kRows * nb * kQ4Block + 15) & ~15u) + (nb * kYStride + nb + kWaves) * sizeof(float);
-    const uint32_t row_bytes = nb * kQ4Block;
-    bool one_pass = row_bytes % 16 == 0 && kGroupsL * row_bytes <= 4 * kWave * 16;
-    for (uint32_t i = 0; i < a.segments; ++i) one_pass = one_pass && (reinterpret_cast<uintptr_t>(a.weights[i]) & 15) == 0;
-    if (one_pass)
-        hipLaunchKernelGGL((q4_0_matvec_kernel<LPR, NBT, true>), dim3(tiles), dim3(kWaves * kWave), lds, stream, a);
-    else
-        hipLaunchKernelGGL((q4_0_matvec_kernel<LPR, NBT, false>), dim3(tiles), dim3(kWaves * kWave), lds, stream, a);
+    const size_t lds = plane_bytes(a.input_width / 32) + (STAGED ? kWaves * stage_bytes(NBT) : 0);
+    hipLaunchKernelGGL((q4_0_matvec_kernel<NBT, KS, STAGED>), dim3(tiles), dim3(kWaves * kWave), lds, stream, a, groups);
     return hipGetLastError();
+}
+
+// Groups of four rows per wavefront: the input's digits cost a workgroup about
+// as much as one group, so the most that leave the card some 448 workgroups
+// whose last round over the CUs is at least nine tenths full.
+uint32_t staged_groups(uint32_t rows) {
+    for (uint32_t groups : {4u, 2u}) {
+        const uint32_t blocks = (rows + 16 * groups - 1) / (16 * groups), rounds = (blocks + 255) / 256;
+        if (blocks >= 448 && 10 * blocks >= 9 * 256 * rounds) return groups;
+    }
+    return 1;
 }
 
 // ---------------------------------------------------------------------------
@@ -391,23 +421,43 @@ __global__ __launch_bounds__(256) void ple_proj_f16_kernel(ATLAS_PP_KPARAMS) {
 
 uint32_t q4_0_matvec_max_input() { return 32 * 4 * 32; }
 
+// Measured on MI355X, us (graph of launches over distinct weights): the vector
+// dot that this replaces, this kernel's first form with one wavefront's four
+// rows loaded by the lanes and staged, and the form kept as it is now:
+//   input  rows          before  lanes  staged  now
+//   1536   256 (gate)    3.12    2.97   3.04    2.50  lanes, KS = 4
+//   2048   1536          2.98    3.78   3.21    2.95  lanes, KS = 4
+//   4096   2048          7.14    5.43   4.67    3.93  lanes, KS = 4
+//   576    3072          3.25    2.72   2.91    2.62  lanes
+//   1536   2560 (QKV)    3.28    3.12   2.95    2.74  staged
+//   1536   12288         5.27    4.98   4.90    4.67  staged
+//   2048   16384         9.45    8.33   6.68    5.99  staged, two groups
+//   3072   18432         11.8    11.8   9.58    9.25  staged
+//   4096   32768         35.1    26.1   20.5    16.8  staged, four groups
+// (4.5 TB/s of the weights at the last.)  More wavefronts per workgroup (8, 12
+// or 16 sharing the digits) were slower at every shape but the last: the
+// barrier waits for all of them.
 hipError_t launch_q4_0_matvec(hipStream_t stream, MatvecArgs a) {
     const uint32_t nb = a.input_width / 32;
-    uint32_t rows = 0;
+    uint64_t rows = 0;
     for (uint32_t i = 0; i < a.segments; ++i) rows += a.width[i];
-    // Lanes per row: 16 (16 rows per workgroup) when that leaves at least
-    // two workgroups per CU and each lane at <= 4 blocks; otherwise 32
-    // (8 rows per workgroup, twice the workgroups for small projections).
-    if (rows >= 16 * 512 && nb <= 64) {
-        if (nb <= 16) return launch_lpr<16, 1>(stream, a);
-        if (nb <= 32) return launch_lpr<16, 2>(stream, a);
-        if (nb <= 48) return launch_lpr<16, 3>(stream, a);
-        return launch_lpr<16, 4>(stream, a);
+    // few rows: spread them, a quarter of a row per wavefront
+    if (rows <= 2048)
+        return nb <= 64 ? launch_shape<1, 4, false>(stream, a, 1) : launch_shape<2, 4, false>(stream, a, 1);
+    // few bytes (nb <= 31 here)
+    if (rows * nb <= 65536)
+        return nb <= 16 ? launch_shape<1, 1, false>(stream, a, 1) : launch_shape<2, 1, false>(stream, a, 1);
+    const uint32_t groups = staged_groups(static_cast<uint32_t>(rows));
+    switch ((nb + kPassBlocks - 1) / kPassBlocks) {
+        case 1: return launch_shape<1, 1, true>(stream, a, groups);
+        case 2: return launch_shape<2, 1, true>(stream, a, groups);
+        case 3: return launch_shape<3, 1, true>(stream, a, groups);
+        case 4: return launch_shape<4, 1, true>(stream, a, groups);
+        case 5: return launch_shape<5, 1, true>(stream, a, groups);
+        case 6: return launch_shape<6, 1, true>(stream, a, groups);
+        case 7: return launch_shape<7, 1, true>(stream, a, groups);
+        default: return launch_shape<8, 1, true>(stream, a, groups);
     }
-    if (nb <= 32) return launch_lpr<32, 1>(stream, a);
-    if (nb <= 64) return launch_lpr<32, 2>(stream, a);
-    if (nb <= 96) return launch_lpr<32, 3>(stream, a);
-    return launch_lpr<32, 4>(stream, a);
 }
 
 uint32_t ple_projection_max_hidden() { return 512 * 8; }
@@ -419,7 +469,7 @@ hipError_t launch_ple_projection_f16(hipStream_t stream, const PleProjArgs& a) {
     constexpr int kRpw = 2;
     const dim3 grid(a.groups * a.width / (4 * kRpw));
     const uint32_t hc = (a.hidden + 511) / 512;
-#define ATLAS_PLE_PROJ(H) hipLaunchKernelGGL((ple_proj_f16_kernel<H, kRpw>), grid, dim3(kWaves * kWave), 0, stream, \
+#define ATLAS_PLE_PROJ(H) hipLaunchKernelGGL((ple_proj_f16_kernel<H, kRpw>), grid, dim3(4 * kWave), 0, stream, \
                                             ATLAS_PP_KARGS(a))
     if (hc <= 1)
         ATLAS_PLE_PROJ(1);
