@@ -652,92 +652,63 @@ __global__ __launch_bounds__(RUN ? 64 * (kRunHelpers + 1) : 64) void rms_reg_ker
     }
 }
 
-// Register-engine configuration: rows per wavefront and the fold of the
-// chunks after the first (exact wave-parallel, or in order from LDS).  Same
-// bits either way.  Measured on MI355X:
-//  * rows < 2048 (decode batches; the row-per-workgroup engine takes over
-//    from 257 or 513 rows, rms_row_engine): one row per wavefront and the
-//    parallel fold -- the in-order chain is fully exposed there (C5 decode
-//    step at 256 rows: 35.9 -> 30.3 us per layer);
+// Register-engine configuration, same bits each way.  Measured on MI355X:
+//  * rows < 2048 (to 512 wide: wider rows are the row-per-workgroup engine's,
+//    rms_row_engine): one row per wavefront, and past the first chunk the
+//    parallel fold as one run with its scans computed ahead by helper
+//    wavefronts (RUN; kRunHelpers): [1, 512] 2.7 us, [256, 512] 3.3;
 //  * rows >= 2048, plain RMSNorm: one row per wavefront, parallel fold
-//    ([4096, 1536]: 11.7 -> 10.6 us);
+//    ([4096, 1536]: 11.7 -> 10.6 us against the fold in order; 13.9 with a
+//    helper), loads staged (10.6 -> 10.2);
 //  * rows >= 2048 with an epilogue operand (residual, add-norm, add-scale):
 //    two rows per wavefront (two wavefronts per SIMD) and the in-order fold
 //    up to the last chunk ([4096, 1536] residual: 16.0 us; one row and the
 //    parallel fold: 16.7; two rows with the parallel fold after the first
-//    chunk, on the later engine: 14.9 against 13.7).
-struct RegConfig {
-    int rows;
-    bool par;
-};
-
-RegConfig pick_reg(uint32_t rows, int mode) {
-    if (rows >= 2048 && mode != kNormPlain) return RegConfig{2, false};
-    return RegConfig{1, true};
-}
-
-// The continuation as one run with its scans computed ahead by helper
-// wavefronts (RUN).  Measured on MI355X: decode batches gain (C5 step at 256
-// rows: 29.5 -> 28.5 us per layer with one helper computing four binades,
-// 27.8 -> 26.8 with two helpers of two binades each, whose scans then land
-// before the head's in-order fold ends; kRunHelpers has the current count);
-// from 2048 rows up the extra wavefronts per row cost more than they hide
-// ([4096, 1536]: 10.3 -> 13.9 us with one helper).
-bool norm_run(uint32_t rows) { return rows < 2048; }
-
+//    chunk, on the later engine: 14.9 against 13.7), loads staged
+//    (16.1 -> 15.5).
 template <int R, int J, int MODE>
-hipError_t launch_reg_rj(hipStream_t s, const NormArgs& a, bool par) {
-    // staged loads from 2048 rows up: plain RMSNorm 10.6 -> 10.2 us and the
-    // residual epilogue 16.1 -> 15.5 us at [4096, 1536]; at decode batches
-    // (256 rows) the extra round trip before the later chunks costs more
-    // (30.2 -> 30.8 us per C5 layer).
-    const bool stage = a.rows >= 2048;
-    const bool run = par && J > 1 && R == 1 && norm_run(a.rows);
-    const size_t lds = run ? (64u * J + 1 + (sizeof(FoldScansLds<4>) + 15) / 16 + 68) * sizeof(f32x4)
-                           : static_cast<size_t>(R) * (a.hidden / 4 + 1) * sizeof(f32x4);
+hipError_t launch_reg_rj(hipStream_t s, const NormArgs& a) {
     const dim3 grid((a.rows + R - 1) / R);
-    if constexpr (R == 1 && J > 1) {
-        if (run) {
+    const size_t lds = static_cast<size_t>(R) * (a.hidden / 4 + 1) * sizeof(f32x4);
+    if constexpr (R == 1 && J == 2) {
+        if (a.rows < 2048) {
+            const size_t run_lds = (64u * J + 1 + (sizeof(FoldScansLds<4>) + 15) / 16 + 68) * sizeof(f32x4);
             hipLaunchKernelGGL((rms_reg_kernel<R, J, MODE, true, false, true>), grid, dim3((kRunHelpers + 1) * kWave),
-                               lds, s, ATLAS_NORM_KARGS(a, 1u, 0u));
+                               run_lds, s, ATLAS_NORM_KARGS(a, 1u, 0u));
             return hipGetLastError();
         }
     }
-    if (par && stage)
-        hipLaunchKernelGGL((rms_reg_kernel<R, J, MODE, true, true, false>), grid, dim3(kWave), lds, s,
-                           ATLAS_NORM_KARGS(a, 1u, 0u));
-    else if (par)
-        hipLaunchKernelGGL((rms_reg_kernel<R, J, MODE, true, false, false>), grid, dim3(kWave), lds, s,
-                           ATLAS_NORM_KARGS(a, 1u, 0u));
-    else if (stage)
-        hipLaunchKernelGGL((rms_reg_kernel<R, J, MODE, false, true, false>), grid, dim3(kWave), lds, s,
-                           ATLAS_NORM_KARGS(a, 1u, 0u));
-    else
-        hipLaunchKernelGGL((rms_reg_kernel<R, J, MODE, false, false, false>), grid, dim3(kWave), lds, s,
-                           ATLAS_NORM_KARGS(a, 1u, 0u));
+    if constexpr (R == 1 && J == 1) {
+        if (a.rows < 2048) {
+            hipLaunchKernelGGL((rms_reg_kernel<R, J, MODE, true, false, false>), grid, dim3(kWave), lds, s,
+                               ATLAS_NORM_KARGS(a, 1u, 0u));
+            return hipGetLastError();
+        }
+    }
+    hipLaunchKernelGGL((rms_reg_kernel<R, J, MODE, R == 1, true, false>), grid, dim3(kWave), lds, s,
+                       ATLAS_NORM_KARGS(a, 1u, 0u));
     return hipGetLastError();
 }
 
 template <int R, int MODE>
-hipError_t launch_reg_r(hipStream_t s, const NormArgs& a, int J, bool par) {
+hipError_t launch_reg_r(hipStream_t s, const NormArgs& a, int J) {
     switch (J) {
-        case 1: return launch_reg_rj<R, 1, MODE>(s, a, par);
-        case 2: return launch_reg_rj<R, 2, MODE>(s, a, par);
-        case 3: return launch_reg_rj<R, 3, MODE>(s, a, par);
-        case 4: return launch_reg_rj<R, 4, MODE>(s, a, par);
-        case 5: return launch_reg_rj<R, 5, MODE>(s, a, par);
-        case 6: return launch_reg_rj<R, 6, MODE>(s, a, par);
-        case 7: return launch_reg_rj<R, 7, MODE>(s, a, par);
-        default: return launch_reg_rj<R, 8, MODE>(s, a, par);
+        case 1: return launch_reg_rj<R, 1, MODE>(s, a);
+        case 2: return launch_reg_rj<R, 2, MODE>(s, a);
+        case 3: return launch_reg_rj<R, 3, MODE>(s, a);
+        case 4: return launch_reg_rj<R, 4, MODE>(s, a);
+        case 5: return launch_reg_rj<R, 5, MODE>(s, a);
+        case 6: return launch_reg_rj<R, 6, MODE>(s, a);
+        case 7: return launch_reg_rj<R, 7, MODE>(s, a);
+        default: return launch_reg_rj<R, 8, MODE>(s, a);
     }
 }
 
 template <int MODE>
 hipError_t launch_reg(hipStream_t s, const NormArgs& a) {
     const int J = static_cast<int>((a.hidden / 4 + 63) / 64);
-    const RegConfig c = pick_reg(a.rows, MODE);
-    if (c.rows == 2) return launch_reg_r<2, MODE>(s, a, J, c.par);
-    return launch_reg_r<1, MODE>(s, a, J, c.par);
+    if (a.rows >= 2048 && MODE != kNormPlain) return launch_reg_r<2, MODE>(s, a, J);
+    return launch_reg_r<1, MODE>(s, a, J);
 }
 
 // Tree engine: two rows per wavefront (rows w and w + G) from 4096 rows up,

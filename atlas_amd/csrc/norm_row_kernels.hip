@@ -1,6 +1,6 @@
 // norm_row_kernels.hip -- RMSNorm engines that give a row to a workgroup, for
 // rows too wide for one wavefront's registers (hidden > 2048) and, in
-// sequential order, for the row counts between a decode batch and a prefill.
+// sequential order, for narrower rows below the prefill's row counts.
 //
 // Semantics and the two reduction orders are norm_kernels.hip's.  A wavefront
 // that holds a 4096-wide row alone keeps 192 registers of data and issues its
@@ -109,34 +109,103 @@ __global__ __launch_bounds__(64 * NW) void rms_row_tree_kernel(ATLAS_NORM_KPARAM
     r.finish(a, base, tid, nv, inverse_rms(s, static_cast<float>(a.hidden), a.epsilon), scale);
 }
 
-// Sequential order, bit for bit, with the fold spread over the wavefronts:
-//  1. every thread squares its columns into LDS; each 256-value block's sum in
-//     any order goes beside them (an estimate: it only chooses binades);
-//  2. wavefront 0 folds the head, the first 256 squares (head_fold_candidates),
-//     while wavefront k >= 1 takes the k-th run of 64 S squares after it, lane
-//     l the S consecutive ones from S l (S / 4 odd: the lanes' 16-byte reads
-//     fall on distinct LDS banks), and computes chunk_scan for the binades that
-//     the running sum can have inside its run by the estimates (at most three,
-//     most often one or two);
-//  3. the running sum goes from wavefront to wavefront, one barrier each; each
-//     walks its run's events with the scans it has (chunk_walk) and falls back
-//     to fold_chunk_exact_from outside them.
-// Bound by that chain at few rows (an event costs ~250 cycles plus S adds, a
-// row has 5 to 9) and by the scans' VALU work at many.
-constexpr int kRowBinades = 3;
+// Sequential order, bit for bit, from segments of 64 squares folded side by
+// side.  Inside a binade a running sum is an integer count of its ulps, and
+// adding a non-negative value raises it by a whole number of ulps that depends
+// on the sum only through its parity (a tie rounds to even).  So a segment
+// that stays in the binade raises every even sum by one amount and every odd
+// sum by another, and a run of such segments is a function of the parity at
+// its start.
+//  1. Every thread squares its columns into LDS; each segment's sum in any
+//     order goes beside them, and every wavefront scans those into estimates
+//     of the segments' starts.
+//  2. Wavefront 0 folds the head, the first 256 squares (head_fold_candidates).
+//     The next PW wavefronts fold every later segment from an even and an odd
+//     start at its estimate, a lane each, 32 segments a pass, and compose the
+//     segments between crossings into runs by a wave scan.  The rest take the
+//     segments that may cross a power of two by the estimates (with a margin of
+//     64 ulps: a segment's in-order sum is within 32 of any other order's):
+//     windows of consecutive starts around the estimate, a lane each.
+//  3. Each window's lane goes on from its fold through the run behind it (one
+//     integer add a group of 32 segments, the binade checked at both ends), and
+//     wavefront 0 from the head through the first run.
+//  4. Every wavefront follows the exact sum from window to window, one readlane
+//     each: about log2(hidden / 256) of them.
+// What the estimates missed -- a start outside its window, more crossings than
+// windows, a binade they put elsewhere -- is folded in order from the exact sum
+// (wavefront 0), and the way goes on with the next window.  Every step is the
+// in-order fold's own adds or provably equals them, so the result is its bit
+// pattern.
+//
+// A sum strays from its estimate by the rounding since the last power of two,
+// about 0.3 sqrt(values) ulps: 32 starts hold it to 1000 values, 64 to the
+// widest row.  With few rows the time is one chain: load, 64 adds behind 16
+// LDS reads, scan, runs, three barriers.  One row of 1536 (residual) 2.9 us,
+// against 3.4 with one wavefront folding whole chunks under helpers' scans
+// (and 2.2 for the tree sum); 4096: 3.4 (5.2 with runs of 4 to 36 float4 a
+// lane); 8192: 4.7 (6.9); [256, 1536] 4.1 (4.6).  Following the sum step by
+// step in wavefront 0, with the runs and windows published as they are: 3.4 at
+// 1536, 4.1 at 4096.
+constexpr uint32_t kSegMargin = 64;
+constexpr uint32_t kNoParity = 0xffffffffu;  // the segment left its binade
+constexpr uint32_t kNoSum = 0xffffffffu;     // no exact sum from this start
+constexpr uint32_t kGroup = 32;              // segments of one parity pass, two lanes each
 
-template <int NW, int Q, int S, int MODE>
-__global__ __launch_bounds__(64 * NW) void rms_row_exact_kernel(ATLAS_NORM_KPARAMS) {
+// Sum over each 16-lane row, in every lane (any order).
+__device__ __forceinline__ float row16_sum(float v) {
+    v += dpp_f32<0xb1, 0xf, false>(v);
+    v += dpp_f32<0x4e, 0xf, false>(v);
+    v += dpp_f32<0x141, 0xf, false>(v);
+    return v + dpp_f32<0x140, 0xf, false>(v);
+}
+
+// Ulps that a run of segments adds to an even (e) and to an odd (o) sum; f
+// marks that the run begins behind a crossing.
+struct ParityRun {
+    uint32_t e, o, f;
+};
+
+template <int CTRL, int ROW_MASK>
+__device__ __forceinline__ void compose_step(ParityRun& b) {
+    const uint32_t ae = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(b.e), CTRL, ROW_MASK, 0xf, false));
+    const uint32_t ao = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(b.o), CTRL, ROW_MASK, 0xf, false));
+    const uint32_t af = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(b.f), CTRL, ROW_MASK, 0xf, false));
+    const uint32_t e = ae + ((ae & 1u) ? b.o : b.e), o = ao + ((ao & 1u) ? b.e : b.o);
+    b.e = b.f ? b.e : e;
+    b.o = b.f ? b.o : o;
+    b.f |= af;
+}
+
+__device__ __forceinline__ float fold_regs_16(const f32x4 (&v)[16], float s) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        s = s + v[i].x;
+        s = s + v[i].y;
+        s = s + v[i].z;
+        s = s + v[i].w;
+    }
+    return s;
+}
+
+template <int NW, int Q, int PW, int HALF, int MODE>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW == 4 && Q == 4 ? 4 : 1)))
+void rms_row_exact_kernel(ATLAS_NORM_KPARAMS) {
     ATLAS_NORM_UNPACK;
-    constexpr uint32_t kBlocks = NW * Q;
-    constexpr uint32_t kRunBlocks = S / 4;
-    __shared__ __align__(16) f32x4 sq4[64 * kBlocks];
-    __shared__ __align__(16) f32x4 head_pad[68];
-    __shared__ float block_sum[kBlocks];
-    __shared__ uint32_t running;
+    constexpr uint32_t kSegs = 4 * NW * Q;  // segments of 16 float4 that the threads hold
+    constexpr int G = (kSegs + 63) / 64;    // registers of one segment per lane
+    constexpr int kCross = NW - 1 - PW;     // wavefronts with windows
+    // windows: two of 32 starts in each of the first HALF such wavefronts, one of 64 in each other
+    constexpr uint32_t kHalves = 2 * HALF, kWindows = kCross + HALF;
+    static_assert(PW >= 1 && HALF >= 0 && HALF <= kCross && kCross >= 1 && G <= 2, "wavefront roles");
+    __shared__ __align__(16) f32x4 sq4[17 * kSegs];  // float4 c at c + c / 16: 16 lanes on distinct banks
+    __shared__ float seg_sum[64 * G];
+    __shared__ __align__(16) u32x4_t runs[kSegs];  // by a run's last segment: ulps from an even, an odd sum; binade
+    __shared__ uint32_t cand[64 * kCross];       // the sum behind a crossing and its run, by the start in the window
+    __shared__ uint32_t window[64];              // a window's first start
+    __shared__ uint32_t first_sum, total;
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(tid >> 6));
-    const uint32_t nv = a.hidden >> 2;
+    const uint32_t nv = a.hidden >> 2, nseg = (nv + 15) / 16;
     const size_t base = static_cast<size_t>(blockIdx.x) * a.hidden;
     RowPart<NW, Q, MODE> r;
     r.load(a, base, tid, nv);
@@ -144,66 +213,207 @@ __global__ __launch_bounds__(64 * NW) void rms_row_exact_kernel(ATLAS_NORM_KPARA
 #pragma unroll
     for (int j = 0; j < Q; ++j) {
         const f32x4 q = r.square(j, tid, nv);
-        const uint32_t block = wave + NW * j;
-        sq4[64u * block + lane] = q;
-        if (j == 0 && wave == 0) head_pad[lane + lane / 16] = q;
-        const float t = wave_sum_any_order_f32((q.x + q.y) + (q.z + q.w));
-        if (lane == 0) block_sum[block] = t;
+        const uint32_t c = r.col(tid, j);
+        sq4[c + c / 16] = q;
+        const float t = row16_sum((q.x + q.y) + (q.z + q.w));
+        if (lane % 16 == 0) seg_sum[c / 16] = t;
     }
-    __syncthreads();  // squares and block sums staged
-    const uint32_t runs = ((nv + 63) / 64 + kRunBlocks - 2) / kRunBlocks;  // ceil((the row's blocks - 1) / kRunBlocks)
-    float run[S];
-    ChunkScan c[kRowBinades];
-    uint32_t e0 = 0, binades = 0;
+    __syncthreads();  // squares and segment sums staged
+
+    float own[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) own[g] = lane + 64u * g < kSegs ? seg_sum[lane + 64u * g] : 0.0f;
+    auto load_segment = [&](f32x4 (&v)[16], uint32_t k) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) v[i] = sq4[17 * k + i];
+    };
+    // est[g]: the estimated start of segment lane + 64 g; cross: the segments
+    // that may leave its binade
+    uint32_t est[G];
+    uint64_t cross[G];
+    auto scan_estimates = [&] {
+        float before = 0.0f;
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            const uint32_t k = lane + 64u * g;
+            const float incl = before + wave_inclusive_scan_f32(own[g]);
+            const float excl = __int_as_float(
+                __builtin_amdgcn_update_dpp(__float_as_int(before), __float_as_int(incl), 0x138, 0xf, 0xf, false));  // wave_shr:1
+            before = readlane_f32(incl, 63);
+            est[g] = __float_as_uint(excl);
+            const bool in = k >= 4 && k < nseg;
+            cross[g] = __builtin_amdgcn_ballot_w64(
+                in && (max(est[g], kSegMargin) - kSegMargin) >> 23 != (__float_as_uint(incl) + kSegMargin) >> 23);
+        }
+    };
+    auto estimate = [&](uint32_t k) {  // any segment's, per lane
+        uint32_t e = static_cast<uint32_t>(__shfl(static_cast<int>(est[0]), static_cast<int>(k & 63u), kWave));
+        if (G > 1) {
+            const uint32_t w = static_cast<uint32_t>(__shfl(static_cast<int>(est[G - 1]), static_cast<int>(k & 63u), kWave));
+            e = k >= 64 ? w : e;
+        }
+        return e;
+    };
+
+    // takes the lowest of the segments that may cross; nseg when there is none
+    auto take_crossing = [&](uint64_t& left0, uint64_t& left1) {
+        const uint32_t p = left0 ? static_cast<uint32_t>(__builtin_ctzll(left0))
+                                 : (left1 ? 64u + static_cast<uint32_t>(__builtin_ctzll(left1)) : nseg);
+        const uint64_t low0 = left0 & (left0 - 1), low1 = left1 & (left1 - 1);
+        left1 = left0 ? left1 : low1;
+        left0 = left0 ? low0 : 0;
+        return p;
+    };
+    // the sum behind the runs from segment pos to the crossing p, from s at pos
+    auto through_runs = [&](uint32_t s, uint32_t pos, uint32_t p, bool& ok) {
+#pragma unroll
+        for (uint32_t k0 = 0; k0 < kSegs; k0 += kGroup) {
+            const uint32_t end = min(p, k0 + kGroup);
+            const bool in = max(pos, k0) < end;
+            const u32x4_t run = runs[in ? end - 1 : 0];
+            const uint32_t to = s + ((s & 1u) ? run.y : run.x);
+            ok = ok && (!in || (((s ^ run.z) | (to ^ run.z)) >> 23) == 0);
+            s = in ? to : s;
+        }
+        return s;
+    };
+
+    uint32_t sum = 0;                // wavefront 0: the bits of the sum behind the head; a window lane's behind its segment
+    uint32_t pos = 4, upto = nseg;  // the run that follows
     if (wave == 0) {
-        const float head = head_fold_candidates(head_pad, lane);
-        if (lane == 0) running = __float_as_uint(head);
-    } else if (wave <= runs) {
-        const uint32_t first = kRunBlocks * (wave - 1) + 1;  // the run's first block
+        const uint32_t head_seg = lane == 0 ? 0u : (lane - 1) / 21 + 1;
+        const uint32_t j = lane == 0 ? 0u : (lane - 1) % 21;
+        f32x4 v[16];
+        load_segment(v, head_seg);  // on its way while the estimates are scanned
+        scan_estimates();
+        // the head, as head_fold_candidates: segment 0 from 0, each of the
+        // next three from the 21 floats around its estimate, then selected
+        uint32_t e[4];
 #pragma unroll
-        for (int i = 0; i < S / 4; ++i) {
-            const uint32_t at = 64u * first + kRunBlocks * lane + i;
-            f32x4 q = sq4[min(at, 64u * kBlocks - 1)];
-            if (kRunBlocks * (NW - 1) >= kBlocks && at >= 64u * kBlocks) q = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-            run[4 * i] = q.x;
-            run[4 * i + 1] = q.y;
-            run[4 * i + 2] = q.z;
-            run[4 * i + 3] = q.w;
+        for (uint32_t k = 1; k < 4; ++k) e[k] = readlane_u32(est[0], k) - 10u;
+        const uint32_t start = head_seg == 0 ? 0u : (head_seg == 1 ? e[1] : (head_seg == 2 ? e[2] : e[3])) + j;
+        const float res = fold_regs_16(v, __uint_as_float(start));
+        sum = readlane_u32(__float_as_uint(res), 0);
+#pragma unroll
+        for (uint32_t k = 1; k < 4; ++k) {
+            const uint32_t at = sum - e[k];
+            if (__builtin_expect(at < 21, 1))
+                sum = readlane_u32(__float_as_uint(res), 21 * k - 20 + at);
+            else
+                sum = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(
+                    __float_as_uint(fold_lds_16(sq4 + 17 * k, __uint_as_float(sum)))));
         }
-        const float mine = lane < kBlocks ? block_sum[lane] : 0.0f;
-        const float before = wave_sum_any_order_f32(lane < first ? mine : 0.0f);
-        const float after = wave_sum_any_order_f32(lane < first + kRunBlocks ? mine : 0.0f);
-        // the in-order sum of <= 8192 squares is within 8192 * 2^-24 < 0.05 %
-        // of the estimate, so these bound its exponent from both sides
-        e0 = __float_as_uint(before * 0.999f) >> 23;
-        const uint32_t e1 = __float_as_uint(after * 1.001f) >> 23;
-        binades = min(e1 - e0 + 1u, static_cast<uint32_t>(kRowBinades));  // wave-uniform
-#pragma unroll
-        for (int b = 0; b < kRowBinades; ++b)
-            if (static_cast<uint32_t>(b) < binades) c[b] = chunk_scan<S>(run, min(max(e0 + b, 27u), 251u));
-    }
-    for (uint32_t k = 1; k <= runs; ++k) {
-        __syncthreads();  // the sum before run k is in `running`
-        if (wave != k) continue;
-        uint32_t sb = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(running));
-        uint32_t l0 = 0;
-#pragma unroll
-        for (int b = 0; b < kRowBinades; ++b) {
-            const uint32_t ex = e0 + b;
-            if (static_cast<uint32_t>(b) < binades && l0 < 64 && (sb >> 23) == ex && ex >= 27 && ex <= 251)
-                l0 = chunk_walk<S>(c[b], run, sb, l0, ex);
+        uint64_t left0 = cross[0], left1 = G > 1 ? cross[G - 1] : 0;
+        upto = take_crossing(left0, left1);
+    } else if (wave <= PW) {
+        f32x4 v[16];
+        load_segment(v, min(kGroup * (wave - 1) + (lane >> 1), nseg - 1));
+        scan_estimates();
+        for (uint32_t k0 = kGroup * (wave - 1); k0 < nseg; k0 += kGroup * PW) {
+            const uint32_t k = k0 + (lane >> 1), kc = min(k, nseg - 1);
+            if (k0 >= kGroup * PW) load_segment(v, kc);  // a later pass
+            const uint32_t start = (estimate(kc) & ~1u) | (lane & 1u);
+            const uint32_t end = __float_as_uint(fold_regs_16(v, __uint_as_float(start)));
+            const bool crosses = ((k < 64 ? cross[0] : cross[G - 1]) >> (k & 63u)) & 1;
+            const uint32_t mine = (start >> 23) == (end >> 23) ? end - start : kNoParity;
+            const uint32_t other = static_cast<uint32_t>(
+                __builtin_amdgcn_update_dpp(0, static_cast<int>(mine), 0xb1, 0xf, 0xf, false));  // the other parity's
+            const bool lost = mine == kNoParity || other == kNoParity;
+            ParityRun run{lane & 1u ? other : mine, lane & 1u ? mine : other, 0u};
+            if (crosses || lost || k < 4) run = ParityRun{0u, 0u, 1u};  // (the head is not part of a run)
+            compose_step<0x112, 0xf>(run);  // row_shr:2, 4, 8: a segment has two lanes
+            compose_step<0x114, 0xf>(run);
+            compose_step<0x118, 0xf>(run);
+            compose_step<0x142, 0xa>(run);
+            compose_step<0x143, 0xc>(run);
+            // (a lost one means a wrong estimate: no run of this pass holds)
+            const bool wrong = __builtin_amdgcn_ballot_w64(lost && !crosses && k >= 4 && k < nseg) != 0;
+            const uint32_t binade = (start >> 23) ^ (wrong ? 0x80u : 0u);
+            if (k < nseg && !(lane & 1u)) runs[k] = u32x4_t{run.e, run.o, binade << 23, 0u};
         }
-        if (l0 < 64) sb = fold_chunk_exact_from<S>(run, sb, l0);
-        if (lane == 0) running = sb;
+    } else {
+        scan_estimates();
+        // this wavefront's windows: crossing number first + i in lanes CW i ..
+        const uint32_t part = wave - 1 - PW;
+        const bool half = part < HALF;
+        const uint32_t first = half ? 2 * part : part + HALF, width = half ? 32u : 64u;
+        uint64_t left0 = cross[0], left1 = G > 1 ? cross[G - 1] : 0;
+        for (uint32_t i = 0; i < first; ++i) take_crossing(left0, left1);
+        const uint32_t p0 = take_crossing(left0, left1), p1 = take_crossing(left0, left1), p2 = take_crossing(left0, left1);
+        const bool second = half && lane >= 32;
+        const uint32_t k = min(second ? p1 : p0, nseg - 1);  // (the last one: a window that no crossing needs)
+        upto = second ? p2 : p1;
+        pos = k + 1;
+        const uint32_t from = estimate(k) - width / 2;
+        if (lane % width == 0) window[first + (second ? 1u : 0u)] = from;
+        sum = __float_as_uint(fold_lds_16(sq4 + 17 * k, __uint_as_float(from + lane % width)));
     }
-    __syncthreads();
-    r.finish(a, base, tid, nv, inverse_rms(__uint_as_float(running), static_cast<float>(a.hidden), a.epsilon), scale);
+    __syncthreads();  // every run published
+    if (wave == 0 || wave > PW) {
+        bool ok = true;
+        const uint32_t to = through_runs(sum, pos, upto, ok);
+        uint32_t* at = wave == 0 ? &first_sum : cand + 64 * (wave - 1 - PW) + lane;
+        if (wave != 0 || lane == 0) *at = ok ? to : kNoSum;
+    }
+    __syncthreads();  // every sum behind a crossing and its run published
+    // every wavefront goes from crossing to crossing
+    uint32_t res[kCross];
+#pragma unroll
+    for (int i = 0; i < kCross; ++i) res[i] = cand[64 * i + lane];
+    const uint32_t windows = window[lane];
+    const uint32_t crossings = __builtin_popcountll(cross[0]) + (G > 1 ? __builtin_popcountll(cross[G - 1]) : 0);
+    uint32_t sb = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(first_sum)), passed = 0;
+    bool on = sb != kNoSum;
+    const bool started = on;
+#pragma unroll
+    for (uint32_t w = 0; w < kWindows; ++w) {
+        const uint32_t width = w < kHalves ? 32 : 64;
+        const uint32_t at = sb - readlane_u32(windows, w);
+        const uint32_t to = w < kHalves ? readlane_u32(res[w / 2], w % 2 * 32 + at % 32) : readlane_u32(res[w - HALF], at % 64);
+        on = on && w < crossings && at < width && to != kNoSum;
+        sb = on ? to : sb;
+        passed += on;
+    }
+    if (__builtin_expect(!started || passed < crossings, 0)) {
+        // a start outside its window, or a run that is not the binade's: folded
+        // in order from the exact sum
+        if (wave == 0) {
+            uint64_t left0 = cross[0], left1 = G > 1 ? cross[G - 1] : 0;
+            uint32_t p = take_crossing(left0, left1), w = 0;  // the next crossing, its number
+            for (; w < passed; ++w) p = take_crossing(left0, left1);
+            uint32_t s = started ? sb : sum, k = started ? p : 4;
+            while (k < nseg) {
+                const uint32_t stop = k < p ? p : k + 1;  // the run before the crossing p, or p itself
+                uint32_t to, behind = stop;
+                bool ok = true;
+                if (k < p) {
+                    to = through_runs(s, k, p, ok);
+                } else {
+                    p = take_crossing(left0, left1);
+                    const uint32_t v = min(w, kWindows - 1), width = v < kHalves ? 32 : 64;
+                    const uint32_t at = s - window[v];
+                    to = cand[(v < kHalves ? 32 * v : 64 * (v - HALF)) + at % width];
+                    ok = w < kWindows && at < width && to != kNoSum;
+                    behind = p;
+                    ++w;
+                }
+                if (ok) {
+                    s = to;
+                    k = behind;
+                }
+                for (; !ok && k < stop; ++k) s = __float_as_uint(fold_lds_16(sq4 + 17 * k, __uint_as_float(s)));
+            }
+        if (lane == 0) total = s;
+        }
+        __syncthreads();
+        sb = total;
+    }
+    r.finish(a, base, tid, nv, inverse_rms(__uint_as_float(sb), static_cast<float>(a.hidden), a.epsilon), scale);
 }
 
-template <int NW, int Q, int S, int MODE>
+template <int NW, int Q, int PW, int HALF, int MODE>
 hipError_t launch_exact(hipStream_t s, const NormArgs& a) {
-    static_assert(64 * NW * Q * 4 >= 256 + 256 && (S / 4) % 2 == 1, "the head and odd runs (LDS banks)");
-    hipLaunchKernelGGL((rms_row_exact_kernel<NW, Q, S, MODE>), dim3(a.rows), dim3(64 * NW), 0, s,
+    hipLaunchKernelGGL((rms_row_exact_kernel<NW, Q, PW, HALF, MODE>), dim3(a.rows), dim3(64 * NW), 0, s,
                        ATLAS_NORM_KARGS(a, 1u, 0u));
     return hipGetLastError();
 }
@@ -215,44 +425,26 @@ hipError_t launch_tree(hipStream_t s, const NormArgs& a) {
     return hipGetLastError();
 }
 
-// Shape of the exact engine: NW Q float4 columns hold the row, and the NW - 1
-// runs of 64 S squares behind the 256 of the head end at or past it
-// (256 + 64 S (NW - 1) values).  NW is a multiple of the four SIMDs (or half
-// of them, two rows then share the SIMDs evenly): with six wavefronts a CU's
-// rows queue on two of its SIMDs (1000 rows of 4096: 19.9 us with six, 11.3
-// with four; 512 rows of 8192: 20.0 with twelve, 12.9 with eight).  Few rows
-// want the work spread (a row's chain is all there is), many rows want few
-// wavefronts per row (the scans of every run are VALU work).  Measured on
-// MI355X, residual epilogue, us (graph of back-to-back launches):
-//   hidden  rows    1      256    1000   4096   wavefront LDS engine before
-//   2304            4.50   6.0    8.3    25.2   13.6 / 17.7 / 29.1 / 45.9
-//   4096            5.2    7.5    11.2   37.0   23.2 / 34.1 / 49.6 / 139.8
-//   8192            6.9    10.1   23.6   79.4   44.7 / 68.6 / 96.0 / 331.9
-//   5120 <8,3,20>   5.8    8.1    17.5   57.5
-//   5120 <4,5,28>   6.2    8.4    16.5   47.9
-//   6144 <8,3,20>   5.9    8.7    19.2   63.3
-//   6144 <4,6,36>   6.9    9.6    19.4   55.0
-//   8192 <4,8,44>   8.3    11.8   26.2   86.1
-// and at hidden <= 2048 between the decode and the prefill engines (RUN below,
-// two rows per wavefront above; row-engine shapes <4,*,*> then <2,*,*>):
-//   1536    rows    512: 5.95 RUN, 5.87    1000: 8.74 RUN, 6.92, 7.11
-//                   1500: 11.4 RUN, 9.7, 8.2    2047: 14.5 RUN, 11.3, 9.3
+// Wavefronts and columns by width, and by rows: up to two workgroups a CU the
+// eight-wavefront shapes win (a thread holds less, and every window has 64
+// starts), past that the four-wavefront ones, which fit more often.  Residual
+// epilogue, us, eight / four wavefronts: [512, 1536] 4.9 / 4.9, [700, 1536]
+// 6.9 / 5.4; [512, 2048] 5.2 / 5.4, [700, 2048] 7.2 / 6.0; [512, 3072] 6.2 / 7.0,
+// [700, 3072] 8.8 / 7.8; [512, 4096] 7.0 / 8.1, [700, 4096] 9.7 / 9.2;
+// [256, 8192] 8.7 / 10.6, [512, 8192] 15.5 / 13.1 (one workgroup a CU there).
+// To 1024 one column a thread leaves nothing to split: [1, 1024] 2.9 / 2.7.
 template <int MODE>
 hipError_t launch_exact_mode(hipStream_t s, const NormArgs& a) {
     const uint32_t h = a.hidden;
-    if (h <= 2048 && a.rows >= 1024) {
-        if (h <= 1536) return launch_exact<2, 3, 20, MODE>(s, a);
-        return launch_exact<2, 4, 28, MODE>(s, a);
-    }
-    if (h <= 1024) return launch_exact<4, 1, 4, MODE>(s, a);
-    if (h <= 2048) return launch_exact<4, 2, 12, MODE>(s, a);
-    if (h <= 2560) return launch_exact<4, 3, 12, MODE>(s, a);
-    if (h <= 3072) return launch_exact<4, 3, 20, MODE>(s, a);
-    if (h <= 4096) return launch_exact<4, 4, 20, MODE>(s, a);
-    if (h <= 6144 && a.rows < 768) return launch_exact<8, 3, 20, MODE>(s, a);
-    if (h <= 5120) return launch_exact<4, 5, 28, MODE>(s, a);
-    if (h <= 6144) return launch_exact<4, 6, 36, MODE>(s, a);
-    return launch_exact<8, 4, 20, MODE>(s, a);
+    const bool few = a.rows <= 512;
+    if (h <= 1024) return launch_exact<4, 1, 1, 2, MODE>(s, a);
+    if (h <= 2048) return few ? launch_exact<8, 1, 1, 0, MODE>(s, a) : launch_exact<4, 2, 1, 1, MODE>(s, a);
+    if (h <= 4096 && few) return launch_exact<8, 2, 2, 0, MODE>(s, a);
+    if (h <= 3072) return launch_exact<4, 3, 1, 2, MODE>(s, a);
+    if (h <= 4096) return launch_exact<4, 4, 1, 2, MODE>(s, a);
+    if (h <= 6144) return launch_exact<8, 3, 3, 1, MODE>(s, a);
+    if (a.rows <= 256) return launch_exact<8, 4, 2, 1, MODE>(s, a);
+    return launch_exact<4, 8, 1, 2, MODE>(s, a);
 }
 
 // [1000, 4096] plain 8.2 us (16.0 with one wavefront per row reading it
@@ -273,10 +465,17 @@ hipError_t launch_mode(hipStream_t s, const NormArgs& a, bool tree) {
 
 }  // namespace
 
+// Sequential order, us by the per-wavefront engine (with its helpers) / by
+// this one, residual: [1, 512] 2.7 / 2.7, [1, 768] 2.9 / 2.8, [1, 320] 2.5 / 2.7;
+// to 512 wide it takes over as rows queue: [700, 512] 3.9 / 4.0, [1000, 512]
+// 4.9 / 4.4, [700, 260] 3.9 / 4.4, [1000, 260] 5.0 / 4.8.  From 2048 rows up to
+// 2048 wide two rows a wavefront keep more loads in flight: [2048, 1536]
+// 9.8 / 9.9, [4096, 1536] 13.6 / 16.8 ([2047, 1536], one row a wavefront:
+// 14.5 / 9.9).  Past 2048 wide there is no other engine to 8192.
 bool rms_row_engine(const NormArgs& a, bool tree) {
     if (a.hidden > 2048) return a.hidden <= 8192;
-    if (tree || a.hidden <= 256 || a.rows >= 2048) return false;
-    return a.rows > (a.hidden > 1536 ? 256u : 512u);
+    if (tree || a.rows >= 2048) return false;
+    return a.hidden > 512 || (a.hidden > 256 && a.rows > 800);
 }
 
 hipError_t launch_rms_norm_row_f32(hipStream_t stream, NormMode mode, bool tree, const NormArgs& a) {

@@ -1,7 +1,7 @@
 """The row-per-workgroup norm engines (f32; hidden 2049 to 8192, and narrower
-rows between the decode and the prefill engines): the exact fold bit for bit
-against the oracle, the tree sum against the operator tolerance, at the edges
-of each workgroup shape and of its runs."""
+rows below the prefill engines): the exact fold bit for bit against the oracle,
+the tree sum against the operator tolerance, at the edges of each workgroup
+shape and of its segments and windows."""
 import cases
 import numpy as np
 import pytest
@@ -10,8 +10,9 @@ from test_gpu_reduction import assert_rms_tolerance, rms_f64
 
 pytestmark = pytest.mark.gpu
 
-# shapes change at 2560, 3072, 4096, 5120 and 6144; runs of 64 S values end at 256 + 64 S k
-EDGES = [2052, 2304, 2556, 2560, 2564, 3072, 3076, 4092, 4096, 4100, 5120, 5124, 6144, 6148, 8188, 8192]
+# shapes change at 1024, 2048, 3072, 4096 and 6144; segments are 64 wide, a pass of runs 2048
+EDGES = [516, 576, 1020, 1024, 1028, 1088, 1536, 2044, 2048, 2052, 2304, 2556, 2564, 3072, 3076, 4092, 4096, 4100, 5124,
+         6144, 6148, 8188, 8192]
 
 
 @pytest.mark.parametrize("hidden", EDGES)
@@ -23,22 +24,37 @@ def test_exact_rows(rt, ora, hidden, mode):
     assert_bits_nan_equal(f"rms_{mode}", cases.rms_gpu(rt, inp, m), cases.rms_oracle(ora, inp, m))
 
 
-@pytest.mark.parametrize("rows,hidden", [(768, 4100), (768, 5120), (768, 5124), (768, 6144)])
-@pytest.mark.parametrize("mode", ["residual", "plain"])
+# rows past the eight-wavefront shapes', and the last and first of each engine
+ROWS = [(513, 1028), (512, 2048), (513, 2048), (513, 2052), (513, 3072), (513, 3076), (513, 4096), (768, 4100), (768, 6144),
+        (256, 8192), (257, 6148), (257, 8192), (1, 512), (1, 516), (800, 260), (801, 260), (800, 512), (801, 512),
+        (2047, 516), (2047, 1536), (2047, 2048), (2048, 516), (2048, 2048)]
+
+
+@pytest.mark.parametrize("rows,hidden", ROWS)
+@pytest.mark.parametrize("mode", ["residual", "plain", "addnorm"])
 def test_exact_rows_many(rt, ora, rows, hidden, mode):
-    inp, m = cases.rms_case(rows, hidden, 1e-6, 9600 + hidden, mode)
+    inp, m = cases.rms_case(rows, hidden, 1e-6, 9600 + rows + hidden, mode)
     inp["x"] = cases.adversarial_rows(rows, hidden, 9700 + hidden)
     assert_bits_nan_equal(f"rms_{mode}", cases.rms_gpu(rt, inp, m), cases.rms_oracle(ora, inp, m))
 
 
-@pytest.mark.parametrize("rows,hidden", [(513, 260), (513, 1024), (513, 1028), (513, 1536), (257, 1540), (257, 2048),
-                                         (512, 1536), (256, 2048), (1023, 576), (1024, 260), (2047, 1536), (1024, 1540),
-                                         (2047, 2048), (2048, 2048)])
-@pytest.mark.parametrize("mode", ["residual", "addnorm"])
-def test_exact_rows_between_engines(rt, ora, rows, hidden, mode):
-    inp, m = cases.rms_case(rows, hidden, 1e-6, 9800 + rows + hidden, mode)
-    inp["x"] = cases.adversarial_rows(rows, hidden, 9900 + hidden)
-    assert_bits_nan_equal(f"rms_{mode}", cases.rms_gpu(rt, inp, m), cases.rms_oracle(ora, inp, m))
+@pytest.mark.parametrize("rows,hidden", [(33, 576), (33, 1536), (513, 1536), (33, 2560), (513, 2560), (33, 4096),
+                                         (513, 4096), (33, 6144), (33, 8192), (257, 8192)])
+def test_exact_rows_more_crossings_than_windows(rt, ora, rows, hidden):
+    # sums that double (row r: every 1 + r % 9 segments), start late, or run into infinity
+    rng = np.random.default_rng(hidden + rows)
+    inp, m = cases.rms_case(rows, hidden, 1e-6, 9900 + hidden, "residual")
+    x = rng.standard_normal((rows, hidden)).astype(np.float32)
+    seg = np.arange(hidden) // 64
+    for r in range(rows):
+        grow = np.exp2(0.5 * (seg // (1 + r % 9)) - 30.0) if r % 4 else np.exp2(0.0 * seg)
+        x[r] *= grow.astype(np.float32)
+        if r % 5 == 2:
+            x[r, : 64 * int(rng.integers(1, hidden // 64))] = 0.0
+        if r % 11 == 7:
+            x[r] *= np.float32(2.0 ** 62)  # finite squares whose sum may overflow
+    inp["x"] = x.reshape(-1)
+    assert_bits_nan_equal("rms_residual", cases.rms_gpu(rt, inp, m), cases.rms_oracle(ora, inp, m))
 
 
 @pytest.mark.parametrize("rows,hidden", [(1, 4096), (701, 2560), (300, 8192)])
