@@ -192,6 +192,12 @@ hipError_t launch_op(hipStream_t s, const float* a, const float* b, float scalar
     return hipGetLastError();
 }
 
+// One 16-byte word a thread, all in flight at once: the link is the bound.
+__global__ __launch_bounds__(256) void host_copy_kernel(const u32x4* from, u32x4* to, uint64_t n) {
+    const uint64_t i = static_cast<uint64_t>(blockIdx.x) * 256 + threadIdx.x;
+    if (i < n) __builtin_nontemporal_store(__builtin_nontemporal_load(from + i), to + i);
+}
+
 }  // namespace
 
 hipError_t launch_elementwise_f32(hipStream_t stream, EltOp op, const float* a, const float* b,
@@ -206,6 +212,14 @@ hipError_t launch_elementwise_f32(hipStream_t stream, EltOp op, const float* a, 
         case kEltScale: return launch_op<kEltScale>(stream, a, b, scalar, out, n);
     }
     return hipErrorInvalidValue;
+}
+
+hipError_t launch_host_copy(hipStream_t stream, const void* from, void* to, size_t bytes) {
+    const uint64_t n = bytes / 16;
+    if (n == 0) return hipSuccess;
+    hipLaunchKernelGGL(host_copy_kernel, dim3(static_cast<uint32_t>((n + 255) / 256)), dim3(256), 0, stream,
+                       static_cast<const u32x4*>(from), static_cast<u32x4*>(to), n);
+    return hipGetLastError();
 }
 
 hipError_t launch_swiglu_f16(hipStream_t stream, const uint16_t* gate, const uint16_t* up, uint16_t* out,

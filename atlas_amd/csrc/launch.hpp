@@ -87,6 +87,9 @@ enum EltOp : int {
 };
 hipError_t launch_elementwise_f32(hipStream_t stream, EltOp op, const float* a, const float* b,
                                   float scalar, float* out, uint64_t n);
+// bytes (a multiple of 16) between a device buffer and pinned host memory,
+// both 16-byte aligned.
+hipError_t launch_host_copy(hipStream_t stream, const void* from, void* to, size_t bytes);
 hipError_t launch_swiglu_f16(hipStream_t stream, const uint16_t* gate, const uint16_t* up,
                              uint16_t* out, uint64_t n);
 hipError_t launch_geglu_offset_f32(hipStream_t stream, const float* gate, const float* ple,
