@@ -2,8 +2,11 @@
 16-byte aligned (16-byte accesses at 4-byte alignment), their tails, in place,
 and the soft cap's shorter divisions over caps and magnitudes at the edges of
 the range that takes them."""
+import ctypes
+
 import numpy as np
 import pytest
+from test_gpu_division import _lib as division_lib
 
 pytestmark = pytest.mark.gpu
 f32 = np.float32
@@ -68,3 +71,13 @@ def test_caps_and_magnitudes(rt, ora, cap):
     assert _same(out.download(x.size), ora.softcap(x, cap))
     rt.free(buf)
     rt.free(out)
+
+
+def test_in_range_division_is_ieee_on_the_exponential_range():
+    # every float from 0.625 to infinity, as test_gpu_division does for the activations
+    counts = (ctypes.c_uint64 * 4)()
+    assert division_lib().atlas_division_check(3, counts) == 0
+    inputs, bad, bad_product, _ = (int(c) for c in counts)
+    assert inputs == 0x7F800000 - int(np.array([0.625], f32).view(np.uint32)[0]) + 1
+    assert bad == 0, f"{bad} inputs differ from the IEEE division"
+    assert bad_product > 1000, bad_product  # planted: no correction step
