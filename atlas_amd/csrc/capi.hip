@@ -9,6 +9,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <chrono>
 #include <cmath>
 #include <cstdarg>
@@ -38,6 +39,7 @@ struct atlas_hip_ctx {
     uint8_t* host_ops_device = nullptr;
     size_t host_ops_bytes = 0;
     hipEvent_t host_ops_event[2] = {};
+    std::atomic<bool> host_ops_busy{false};
     std::string last_error;
     atlas_hip_telemetry tel{};
 };
@@ -967,9 +969,9 @@ namespace {
 constexpr size_t kHostOpsMax = size_t{16} << 20;
 constexpr size_t kHostOpsMin = size_t{1} << 20;
 
-// Makes the context's buffers hold `bytes`; false: the call allocates its own.
+// Makes the context's buffers hold `bytes` (at most kHostOpsMax); false: the call
+// allocates its own.
 bool reserve_host_ops(atlas_hip_ctx* ctx, size_t bytes) {
-    if (bytes > kHostOpsMax) return false;
     if (bytes <= ctx->host_ops_bytes) return true;
     size_t size = kHostOpsMin;
     while (size < bytes) size *= 2;
@@ -994,7 +996,8 @@ bool reserve_host_ops(atlas_hip_ctx* ctx, size_t bytes) {
 //
 // A call that fits is served from the context's buffers: the inputs are copied
 // to pinned memory side by side and go up in one transfer, the output comes
-// down in one, and the host waits once.  Against a buffer for each operand with
+// down in one, and the host waits once.  A call that finds the buffers taken by
+// another thread's allocates its own.  Against a buffer for each operand with
 // a transfer from the caller's pageable memory and a wait each, us a call: silu
 // of 256 bytes 53 -> 30, of 295 KB 62 -> 48, of 2.1 MB 304 -> 203, add of 4.2 MB
 // 660 -> 490; RMSNorm and RoPE of [128, 576] 77 and 90 -> 50.  Sending an input
@@ -1002,20 +1005,23 @@ bool reserve_host_ops(atlas_hip_ctx* ctx, size_t bytes) {
 // against 94): each transfer costs more than it hides.
 class Scratch {
 public:
-    Scratch(atlas_hip_ctx* c, std::initializer_list<size_t> operand_bytes) : ctx_(c), before_(c->tel.resident_bytes) {
+    Scratch(atlas_hip_ctx* c, std::initializer_list<size_t> operand_bytes) : ctx_(c) {
         size_t total = 0;
         bool fits = !c->capturing;
         for (const size_t bytes : operand_bytes) {
             fits = fits && bytes <= kHostOpsMax;
             total += fits ? padded(bytes) : 0;
         }
-        pooled_ = fits && reserve_host_ops(c, total);
+        if (!fits || total > kHostOpsMax || c->host_ops_busy.exchange(true)) return;
+        pooled_ = reserve_host_ops(c, total);
+        if (!pooled_) c->host_ops_busy = false;
     }
     ~Scratch() {
-        if (pooled_)
-            ctx_->tel.resident_bytes = before_;
-        else
-            for (int i = 0; i < n_; ++i) atlas_hip_free(ctx_, ptrs_[i]);
+        if (pooled_) {
+            ctx_->tel.resident_bytes -= taken_;
+            ctx_->host_ops_busy = false;
+        }
+        for (int i = 0; i < n_; ++i) atlas_hip_free(ctx_, ptrs_[i]);
     }
     Scratch(const Scratch&) = delete;
     Scratch& operator=(const Scratch&) = delete;
@@ -1080,6 +1086,7 @@ private:
     void* take(size_t bytes) {
         void* p = ctx_->host_ops_device + used_;
         used_ += padded(bytes);
+        taken_ += bytes;
         ctx_->tel.allocations += 1;
         ctx_->tel.resident_bytes += bytes;
         if (ctx_->tel.resident_bytes > ctx_->tel.peak_resident_bytes)
@@ -1120,7 +1127,7 @@ private:
 
     atlas_hip_ctx* ctx_;
     bool pooled_ = false;
-    size_t before_, used_ = 0, in_bytes_ = 0, out_at_ = 0;
+    size_t taken_ = 0, used_ = 0, in_bytes_ = 0, out_at_ = 0;
     void* ptrs_[8] = {};
     int n_ = 0;
 };

@@ -1,6 +1,8 @@
 """The host-slice operators over the context's buffers: operands from one value
 to past what the context keeps, in changing order, against the formulas of
 the operators on the CPU; telemetry and refusals as with a buffer per operand."""
+import threading
+
 import numpy as np
 import pytest
 from atlas_amd import NeuralOps, OperatorError
@@ -72,3 +74,24 @@ def test_telemetry_and_refusals():
     finally:
         ops.rt.graph_destroy(ops.rt.graph_end())
     assert np.array_equal(ops.add(x, x)[0], x + x)
+
+
+def test_threads_on_one_context(ops):
+    """Calls that overlap take the kept buffers one at a time and allocate
+    otherwise: each gets its own result."""
+    rng = np.random.default_rng(9)
+    inputs = [rng.standard_normal(n, dtype=np.float32) for n in (1000, 70001, 300000, 64)]
+    wrong = []
+
+    def work(x):
+        for _ in range(20):
+            got = ops.add(x, x)[0]
+            if not np.array_equal(got, x + x):
+                wrong.append(x.size)
+
+    threads = [threading.Thread(target=work, args=(x,)) for x in inputs]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert wrong == []
