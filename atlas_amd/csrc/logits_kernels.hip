@@ -43,34 +43,36 @@ __device__ __forceinline__ uint64_t argmax_key(float v, uint32_t index) {
 
 __device__ __forceinline__ uint64_t max_u64(uint64_t a, uint64_t b) { return a > b ? a : b; }
 
-// The cap and what a wavefront's plain values need of it: rcp = RN(1 / cap).
+// The cap, and what a wavefront's plain values need of it: rcp = RN(1 / cap),
+// formed on the host; 0 for a cap outside [2^-20, 2^20].
 struct SoftCap {
     float cap, rcp;
-    bool plain;  // cap in [2^-20, 2^20]
 };
 
-__device__ __forceinline__ SoftCap soft_cap(float cap) {
-    return {cap, fdiv_rn(1.0f, cap), cap >= 0x1p-20f && cap <= 0x1p20f};
-}
+SoftCap soft_cap(float cap) { return {cap, cap >= 0x1p-20f && cap <= 0x1p20f ? 1.0f / cap : 0.0f}; }
 
 // cap * tanh(v / cap) for the values of one lane, with the bits of the IEEE
 // steps (fdiv_rn, tanh_series_abs, tanh_exp_abs) throughout.  The series is
 // evaluated for every value; the exponential only when some lane of the
 // wavefront needs it (a wave-uniform branch), then selected per value.  Bound
-// by this arithmetic where logits reach the exponential (|v| >= 0.625 cap),
-// so wavefronts whose |v| all lie in [2^-70, 2^60] -- ordinary logits; an
-// exact zero, an infinity or a NaN row sends the wavefront to the full form --
-// take shorter divisions:
-//  * v / cap: q0 = v rcp is within 1.5 ulp of the quotient; q1 = fma(v - q0
-//    cap, rcp, q0) within half an ulp and a few 2^-22 of one, so faithful; and
-//    q2 = fma(v - q1 cap, rcp, q1), with the residual exact (no operand or
-//    product comes near the subnormals) and rcp correctly rounded, is the
-//    correctly rounded quotient (Markstein 1990).  Five operations against the
-//    division's eleven;
-//  * 2 / (e^{2a} + 1): tanh_exp_abs_with, enumerated equal over its domain.
+// by this arithmetic where logits reach the exponential (|v| >= 0.625 cap), so
+// both divisions are shorter ones where that is exact:
+//  * v / cap in wavefronts whose |v| all lie in [2^-70, 2^60] -- ordinary
+//    logits; an exact zero, a mask's -inf or lowest float sends the wavefront
+//    to the IEEE division: q0 = v rcp is within 1.5 ulp of the quotient; q1 =
+//    fma(v - q0 cap, rcp, q0) within half an ulp and a few 2^-22 of one, so
+//    faithful; and q2 = fma(v - q1 cap, rcp, q1), with the residual exact (no
+//    operand or product comes near the subnormals) and rcp correctly rounded,
+//    is the correctly rounded quotient (Markstein 1990).  Five operations
+//    against the division's eleven;
+//  * 2 / (e^{2a} + 1): tanh_exp_abs_with, enumerated equal over its whole
+//    domain, for every wavefront.
 // With wave_key below, soft cap + argmax of [256, 262144] at logits of standard
-// deviation 8 and cap 30: 135 -> 98 us (the soft cap alone 119 -> 92; at
-// deviation 1, where no value reaches the exponential, 91.8 -> 90.7).
+// deviation 8 and cap 30: 135 -> 95 us (the soft cap alone 119 -> 93, and with
+// 2 % of the values at -inf 122 -> 103; 124 when such a wavefront took both
+// long divisions behind the range test, which [256, 32000], a cache-resident
+// batch, showed most: 16.6 -> 20.0, now 15.5); at deviation 1, where no value
+// reaches the exponential, 93 both ways.
 template <int N>
 __device__ __forceinline__ void softcap_lanes(float (&v)[N], const SoftCap& k) {
     float hi = __builtin_fabsf(v[0]), lo = hi;
@@ -80,38 +82,27 @@ __device__ __forceinline__ void softcap_lanes(float (&v)[N], const SoftCap& k) {
         lo = fminf(lo, __builtin_fabsf(v[i]));
     }
     float a[N], r[N];
-    if (k.plain && __builtin_amdgcn_ballot_w64(!(hi <= 0x1p60f && lo >= 0x1p-70f)) == 0) {
-        // NaN among plain values: max and min skip it, every step below
-        // propagates it and the range test leaves it to the series
+    // NaN among plain values: max and min skip it, every step propagates it
+    // and the range test below leaves it to the series
+    if (k.rcp != 0.0f && __builtin_amdgcn_ballot_w64(!(hi <= 0x1p60f && lo >= 0x1p-70f)) == 0) {
 #pragma unroll
         for (int i = 0; i < N; ++i) {
             const float q0 = v[i] * k.rcp;
             const float q1 = __builtin_fmaf(__builtin_fmaf(-q0, k.cap, v[i]), k.rcp, q0);
             a[i] = __builtin_fabsf(__builtin_fmaf(__builtin_fmaf(-q1, k.cap, v[i]), k.rcp, q1));
-            r[i] = tanh_series_abs(a[i]);
-        }
-        // the quotient rounds monotonically: below 0.6249 cap none reaches 0.625
-        if (__builtin_amdgcn_ballot_w64(hi >= 0.6249f * k.cap) != 0) {
-#pragma unroll
-            for (int i = 0; i < N; ++i) {
-                const float big = tanh_exp_abs_with<DivPositive>(a[i]);
-                r[i] = a[i] >= 0.625f ? big : r[i];
-            }
         }
     } else {
-        bool need_exp = false;
+#pragma unroll
+        for (int i = 0; i < N; ++i) a[i] = __builtin_fabsf(fdiv_rn(v[i], k.cap));
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i) r[i] = tanh_series_abs(a[i]);
+    // the quotient rounds monotonically: below 0.6249 cap none reaches 0.625
+    if (__builtin_amdgcn_ballot_w64(hi >= 0.6249f * k.cap) != 0) {
 #pragma unroll
         for (int i = 0; i < N; ++i) {
-            a[i] = __builtin_fabsf(fdiv_rn(v[i], k.cap));
-            need_exp = need_exp || !tanh_series_range(a[i]);
-            r[i] = tanh_series_abs(a[i]);
-        }
-        if (__builtin_amdgcn_ballot_w64(need_exp) != 0) {
-#pragma unroll
-            for (int i = 0; i < N; ++i) {
-                const float big = tanh_exp_abs(a[i]);
-                r[i] = tanh_series_range(a[i]) ? r[i] : big;
-            }
+            const float big = tanh_exp_abs_with<DivPositive>(a[i]);
+            r[i] = a[i] >= 0.625f ? big : r[i];
         }
     }
     // cap > 0: the quotient's sign is v's
@@ -194,13 +185,13 @@ typedef f32x4 f32x4_row __attribute__((aligned(4)));
 
 template <bool CAP, bool ARG, int U>
 __global__ __launch_bounds__(kLogitThreads) void logits_vec_kernel(const float* in, float* out, uint32_t count,
-                                                                   uint32_t per_block, float cap, uint64_t* slots,
-                                                                   uint32_t* selected) {
+                                                                   uint32_t per_block, float cap, float rcp,
+                                                                   uint64_t* slots, uint32_t* selected) {
     const uint32_t row = blockIdx.y;
     const uint64_t base = static_cast<uint64_t>(row) * count;
     const uint32_t first = blockIdx.x * per_block;
     const uint32_t last = count - first < per_block ? count : first + per_block;
-    const SoftCap k = soft_cap(CAP ? cap : 1.0f);
+    const SoftCap k{cap, rcp};
     const uint32_t wave = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(threadIdx.x / kWave));
     uint64_t key = 0;
     for (uint32_t begin = first; begin < last; begin += kLogitThreads * 4 * U) {
@@ -254,13 +245,13 @@ __global__ __launch_bounds__(kLogitThreads) void logits_vec_kernel(const float* 
 // Rows of fewer than 4 values: one value per thread per step.
 template <bool CAP, bool ARG>
 __global__ __launch_bounds__(kLogitThreads) void logits_scalar_kernel(const float* in, float* out, uint32_t count,
-                                                                      uint32_t per_block, float cap, uint64_t* slots,
-                                                                      uint32_t* selected) {
+                                                                      uint32_t per_block, float cap, float rcp,
+                                                                      uint64_t* slots, uint32_t* selected) {
     const uint32_t row = blockIdx.y;
     const uint64_t base = static_cast<uint64_t>(row) * count;
     const uint32_t begin = blockIdx.x * per_block;
     const uint32_t end = count - begin < per_block ? count : begin + per_block;
-    const SoftCap k = soft_cap(CAP ? cap : 1.0f);
+    const SoftCap k{cap, rcp};
     uint64_t key = 0;
     for (uint32_t i = begin + threadIdx.x; i < end; i += kLogitThreads) {
         float x[1] = {in[base + i]};
@@ -314,6 +305,7 @@ uint32_t row_launch_rows(uint32_t blocks, uint32_t slot_count) {
 template <bool CAP, bool ARG>
 hipError_t launch_rows(hipStream_t stream, const float* in, float* out, uint32_t* selected, uint32_t rows,
                        uint32_t count, float cap, uint64_t* slots, uint32_t slot_count) {
+    const SoftCap k = soft_cap(cap);
     const RowSplit split = row_split(count >= 4, rows, count);
     const bool vec = split.vec, wide = split.wide;
     const uint32_t blocks = split.blocks, per_block = split.per_block;
@@ -326,13 +318,13 @@ hipError_t launch_rows(hipStream_t stream, const float* in, float* out, uint32_t
         uint32_t* rsel = ARG ? selected + r0 : nullptr;
         if (vec && wide)
             hipLaunchKernelGGL((logits_vec_kernel<CAP, ARG, 4>), grid, dim3(kLogitThreads), 0, stream, rin, rout,
-                               count, per_block, cap, slots, rsel);
+                               count, per_block, k.cap, k.rcp, slots, rsel);
         else if (vec)
             hipLaunchKernelGGL((logits_vec_kernel<CAP, ARG, 1>), grid, dim3(kLogitThreads), 0, stream, rin, rout,
-                               count, per_block, cap, slots, rsel);
+                               count, per_block, k.cap, k.rcp, slots, rsel);
         else
             hipLaunchKernelGGL((logits_scalar_kernel<CAP, ARG>), grid, dim3(kLogitThreads), 0, stream, rin, rout,
-                               count, per_block, cap, slots, rsel);
+                               count, per_block, k.cap, k.rcp, slots, rsel);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
         if (ARG && blocks > 1) {
@@ -348,9 +340,9 @@ hipError_t launch_rows(hipStream_t stream, const float* in, float* out, uint32_t
 
 // Soft cap of a flat array: grid-stride float4 body plus a scalar tail.
 __global__ __launch_bounds__(kLogitThreads) void softcap_vec_kernel(const float* in, float* out, uint64_t n4,
-                                                                    float cap) {
+                                                                    float cap, float rcp) {
     const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
-    const SoftCap k = soft_cap(cap);
+    const SoftCap k{cap, rcp};
     for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n4; i += stride) {
         const f32x4 v = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(in) + i);
         float x[4] = {v.x, v.y, v.z, v.w};
@@ -360,9 +352,9 @@ __global__ __launch_bounds__(kLogitThreads) void softcap_vec_kernel(const float*
 }
 
 __global__ __launch_bounds__(kLogitThreads) void softcap_scalar_kernel(const float* in, float* out, uint64_t begin,
-                                                                       uint64_t n, float cap) {
+                                                                       uint64_t n, float cap, float rcp) {
     const uint64_t stride = static_cast<uint64_t>(gridDim.x) * blockDim.x;
-    const SoftCap k = soft_cap(cap);
+    const SoftCap k{cap, rcp};
     for (uint64_t i = begin + static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += stride) {
         float x[1] = {in[i]};
         softcap_lanes(x, k);
@@ -419,14 +411,16 @@ hipError_t argmax_scratch_address(void** ptr) {
 hipError_t launch_softcap_f32(hipStream_t stream, const float* in, float* out, uint64_t n, float cap) {
     const bool vec = (reinterpret_cast<uintptr_t>(in) & 15) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0;
     const uint64_t n4 = vec ? n / 4 : 0;
+    const SoftCap k = soft_cap(cap);
     if (n4) {
-        hipLaunchKernelGGL(softcap_vec_kernel, dim3(grid_for(n4)), dim3(kLogitThreads), 0, stream, in, out, n4, cap);
+        hipLaunchKernelGGL(softcap_vec_kernel, dim3(grid_for(n4)), dim3(kLogitThreads), 0, stream, in, out, n4, k.cap,
+                           k.rcp);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
     if (n4 * 4 < n) {
         hipLaunchKernelGGL(softcap_scalar_kernel, dim3(grid_for(n - n4 * 4)), dim3(kLogitThreads), 0, stream, in, out,
-                           n4 * 4, n, cap);
+                           n4 * 4, n, k.cap, k.rcp);
         return hipGetLastError();
     }
     return hipSuccess;

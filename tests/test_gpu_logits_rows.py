@@ -73,6 +73,37 @@ def test_caps_and_magnitudes(rt, ora, cap):
     rt.free(out)
 
 
+# a wavefront meets the IEEE division through any of its values: exact zeros,
+# a mask's -inf or lowest float, infinities, NaN and subnormals beside ordinary
+# logits, in rows of one value a thread, of one and of four float4 a thread
+SPECIAL = np.array([0.0, -0.0, -np.inf, np.inf, np.finfo(f32).min, np.finfo(f32).max, np.nan, 1e-45, -1e-40, 2.0 ** -71],
+                   f32)
+
+
+@pytest.mark.parametrize("rows,count", [(5, 3), (3, 259), (64, 4096), (1024, 4096), (1031, 4099)])
+@pytest.mark.parametrize("std", [1.0, 8.0])
+def test_special_values(rt, ora, rows, count, std):
+    r = np.random.default_rng(rows + count)
+    x = (r.standard_normal((rows, count)) * std).astype(f32)
+    for i in range(rows):
+        if i % 3 == 1:  # one special value in the row
+            x[i, r.integers(count)] = SPECIAL[(i // 3) % len(SPECIAL)]
+        elif i % 3 == 2:  # a masked row
+            x[i, r.random(count) < 0.5] = SPECIAL[2 + (i // 3) % 3]
+    x = x.reshape(-1)
+    exp_c, exp_s = ora.softcap_argmax_rows(x, rows, count, 30.0)
+    src, dst, sel = rt.upload(x), rt.empty(x.size), rt.empty(rows, np.uint32)
+    rt.softcap_argmax(src, dst, sel, rows, count, 30.0)
+    rt.sync()
+    assert _same(dst.download(x.size), exp_c)
+    assert np.array_equal(sel.download(rows, np.uint32), exp_s)
+    rt.softcap(src, src, x.size, 30.0)
+    rt.sync()
+    assert _same(src.download(x.size), exp_c)
+    for b in (src, dst, sel):
+        rt.free(b)
+
+
 def test_in_range_division_is_ieee_on_the_exponential_range():
     # every float from 0.625 to infinity, as test_gpu_division does for the activations
     counts = (ctypes.c_uint64 * 4)()
