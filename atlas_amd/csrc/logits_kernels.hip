@@ -195,6 +195,9 @@ __global__ __launch_bounds__(kLogitThreads) void logits_vec_kernel(const float* 
     const uint32_t wave = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(threadIdx.x / kWave));
     uint64_t key = 0;
     for (uint32_t begin = first; begin < last; begin += kLogitThreads * 4 * U) {
+        // short rows: no value of this step is this wavefront's (with U = 4 the
+        // test costs more registers than it saves)
+        if (U == 1 && begin + wave * (kWave * 4) >= last) break;
         float x[4 * U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -242,7 +245,7 @@ __global__ __launch_bounds__(kLogitThreads) void logits_vec_kernel(const float* 
     if (ARG) publish_key<true>(key, row, slots, selected);
 }
 
-// Rows of fewer than 4 values: one value per thread per step.
+// Rows of few values (launch_split): one value per thread per step.
 template <bool CAP, bool ARG>
 __global__ __launch_bounds__(kLogitThreads) void logits_scalar_kernel(const float* in, float* out, uint32_t count,
                                                                       uint32_t per_block, float cap, float rcp,
@@ -269,14 +272,14 @@ struct RowSplit {
     uint32_t blocks, per_block;
 };
 
-RowSplit row_split(bool vec, uint32_t rows, uint32_t count) {
+RowSplit row_split(bool vec, bool wide, uint32_t rows, uint32_t count) {
     RowSplit r;
     r.vec = vec;
     // large batches: steps of 4096 values; a single row: 1024, for more
     // workgroups in flight.  At most kArgmaxSlotsPerRow workgroups per row:
     // longer rows give each workgroup several steps.
-    r.wide = static_cast<uint64_t>(rows) * count >= (1u << 22);
-    const uint32_t step = r.vec && r.wide ? 4096u : 1024u;
+    r.wide = vec && wide && static_cast<uint64_t>(rows) * count >= (1u << 22);
+    const uint32_t step = r.wide ? 4096u : 1024u;
     r.blocks = (count + step - 1) / step;
     r.per_block = step;
     if (r.blocks > kArgmaxSlotsPerRow) {
@@ -286,14 +289,34 @@ RowSplit row_split(bool vec, uint32_t rows, uint32_t count) {
     return r;
 }
 
+bool aligned_rows(const float* in, const float* out, uint32_t count) {
+    return count % 4 == 0 && (reinterpret_cast<uintptr_t>(in) & 15) == 0 &&
+           (!out || (reinterpret_cast<uintptr_t>(out) & 15) == 0);
+}
+
 // The split that the no-allocation entry point's limit is stated in: rows
 // that are not a multiple of 4 values, or not 16-byte aligned, count their
 // workgroups in steps of 1024 values at any batch size.  The launch itself
 // needs at most as many.
 RowSplit limit_split(const float* in, const float* out, uint32_t rows, uint32_t count) {
-    return row_split(count % 4 == 0 && (reinterpret_cast<uintptr_t>(in) & 15) == 0 &&
-                         (!out || (reinterpret_cast<uintptr_t>(out) & 15) == 0),
-                     rows, count);
+    const bool aligned = aligned_rows(in, out, count);
+    return row_split(aligned, aligned, rows, count);
+}
+
+// The split of a launch.  Aligned rows take float4 steps from 4 values on, and
+// so does an argmax of any row.  The soft cap of unaligned rows computes every
+// value that its float4 repeat: short rows go one value a thread, and rows that
+// would fill less than 0.6 of their wide steps take narrow ones.  Soft cap +
+// argmax of [4000, n], us, one value a thread / narrow / wide:
+//   n = 5     5.5 / 6.4 / -         129   6.9 / 7.5 / -       ([1000, 385] 4.5 / 4.9)
+//   n = 513   10.7 / 8.8 / -        1537  27 / 18.5 / 22.8    (masked 27 / 19.3 / 29)
+//   n = 4097  52 / 36 / 42 (masked 51 / 36 / 50)
+//   n = 8193  96 / 65 / 58 (masked 93 / 64 / 70)              12001  135 / 88 / 76
+template <bool CAP>
+RowSplit launch_split(const float* in, const float* out, uint32_t rows, uint32_t count) {
+    const bool loose = CAP && !aligned_rows(in, out, count);
+    const uint64_t wide_steps = (static_cast<uint64_t>(count) + 4095) / 4096 * 4096;
+    return row_split(count >= (loose ? 512u : 4u), !loose || 5ull * count >= 3 * wide_steps, rows, count);
 }
 
 // Rows one launch can cover with `slot_count` workspace slots (a row split
@@ -306,7 +329,7 @@ template <bool CAP, bool ARG>
 hipError_t launch_rows(hipStream_t stream, const float* in, float* out, uint32_t* selected, uint32_t rows,
                        uint32_t count, float cap, uint64_t* slots, uint32_t slot_count) {
     const SoftCap k = soft_cap(cap);
-    const RowSplit split = row_split(count >= 4, rows, count);
+    const RowSplit split = launch_split<CAP>(in, out, rows, count);
     const bool vec = split.vec, wide = split.wide;
     const uint32_t blocks = split.blocks, per_block = split.per_block;
     const uint32_t rows_per_launch = row_launch_rows(blocks, slot_count);

@@ -28,7 +28,11 @@ def _same(got, exp):
 
 
 @pytest.mark.parametrize("rows,count", [(1, 3), (5, 4), (7, 5), (9, 7), (3, 1023), (3, 1026), (2, 4095), (2, 4099),
-                                        (1, 32001), (130, 32001), (85, 50257), (3, 1400005)])
+                                        (1, 32001), (130, 32001), (85, 50257), (3, 1400005),
+                                        # where the launch form changes: 512 values, 2^22 in all, steps
+                                        # of 4096 that are 0.6 full
+                                        (4, 511), (4, 513), (9000, 509), (8300, 515), (1710, 2457), (1710, 2458),
+                                        (1025, 4097), (33, 512), (20, 260), (70000, 5)])
 @pytest.mark.parametrize("offset,in_place", [(0, False), (4, False), (12, True)])
 def test_rows(rt, ora, rows, count, offset, in_place):
     x = _rows(rows + count, rows, count, 8.0)
