@@ -426,7 +426,7 @@ uint32_t q4_0_matvec_max_input() { return 32 * 4 * 32; }
 // rows loaded by the lanes and staged, and the form kept as it is now:
 //   input  rows          before  lanes  staged  now
 //   1536   256 (gate)    3.12    2.97   3.04    2.50  lanes, KS = 4
-//   2048   1536          2.98    3.78   3.21    2.95  lanes, KS = 4
+//   2048   1536          2.98    3.78   3.21    2.95  lanes, KS = 2
 //   4096   2048          7.14    5.43   4.67    3.93  lanes, KS = 4
 //   576    3072          3.25    2.72   2.91    2.62  lanes
 //   1536   2560 (QKV)    3.28    3.12   2.95    2.74  staged
@@ -434,19 +434,44 @@ uint32_t q4_0_matvec_max_input() { return 32 * 4 * 32; }
 //   2048   16384         9.45    8.33   6.68    5.99  staged, two groups
 //   3072   18432         11.8    11.8   9.58    9.25  staged
 //   4096   32768         35.1    26.1   20.5    16.8  staged, four groups
-// (4.5 TB/s of the weights at the last.)  More wavefronts per workgroup (8, 12
-// or 16 sharing the digits) were slower at every shape but the last: the
-// barrier waits for all of them.
+// (4.5 TB/s of the weights at the last.)  A row is split between four or two
+// wavefronts while that leaves each CU one workgroup (1024 and 2048 rows) and
+// the row has the passes to split; from there on a second round of workgroups
+// costs more than the split saves.  One projection, us: the vector dot / four
+// wavefronts a row / two / one, lanes / one, staged:
+//   input  rows   vector  KS=4   KS=2   lanes  staged
+//   512    1024   3.02    2.99   2.98   2.83   2.90
+//   512    2048   3.21    3.31   3.15   2.99   3.12
+//   768    16     2.88    2.84   2.59   2.61   2.68
+//   768    1024   3.06    3.04   3.14   3.08   3.30
+//   768    2048   3.21    3.39   3.26   3.14   3.39
+//   1024   4096   3.89    4.23   3.66   3.33   3.56
+//   544    6144    -       -      -     4.04   3.75
+//   1024   6144   4.43    5.02   4.10   4.00   3.97
+//   32     131072  -       -      -     10.9   7.57
+//   1536   1024   3.49    3.12   3.23   3.47   3.29
+//   1536   2048   3.77    3.51   3.27   3.58   3.32
+//   3072   1024   3.92    3.46   3.75   4.48   4.00
+//   3072   1088   4.05    4.33   3.77   4.42   4.01
+//   3072   2048   4.09    4.49   3.87   4.51   4.03
+//   3072   2560   4.86    5.21   4.63   4.59   4.12
+//   4096   1024   7.31    4.14   4.78   5.89   5.07
+//   4096   2048   7.39    4.88   4.90   5.92   5.08
+// More wavefronts per workgroup (8, 12 or 16 sharing the digits) were slower at
+// every shape but 4096 -> 32768: the barrier waits for all of them.
 hipError_t launch_q4_0_matvec(hipStream_t stream, MatvecArgs a) {
     const uint32_t nb = a.input_width / 32;
     uint64_t rows = 0;
     for (uint32_t i = 0; i < a.segments; ++i) rows += a.width[i];
-    // few rows: spread them, a quarter of a row per wavefront
-    if (rows <= 2048)
+    const bool few_bytes = rows <= 4096 || rows * nb <= 65536;  // the staged form pipelines more than these give it
+    if (nb <= 16 && few_bytes) return launch_shape<1, 1, false>(stream, a, 1);
+    if (rows <= 1024 && (nb > 32 || rows > 32))
         return nb <= 64 ? launch_shape<1, 4, false>(stream, a, 1) : launch_shape<2, 4, false>(stream, a, 1);
-    // few bytes (nb <= 31 here)
-    if (rows * nb <= 65536)
-        return nb <= 16 ? launch_shape<1, 1, false>(stream, a, 1) : launch_shape<2, 1, false>(stream, a, 1);
+    if (nb <= 32 && few_bytes) return launch_shape<2, 1, false>(stream, a, 1);
+    if (rows <= 2048) {
+        if (nb <= 64) return launch_shape<2, 2, false>(stream, a, 1);
+        return nb <= 96 ? launch_shape<3, 2, false>(stream, a, 1) : launch_shape<4, 2, false>(stream, a, 1);
+    }
     const uint32_t groups = staged_groups(static_cast<uint32_t>(rows));
     switch ((nb + kPassBlocks - 1) / kPassBlocks) {
         case 1: return launch_shape<1, 1, true>(stream, a, groups);

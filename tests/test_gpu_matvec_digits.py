@@ -36,7 +36,10 @@ def _check(ora, got, x, W, w, n, rows):
 @pytest.mark.parametrize("n,rows", [
     (32, 1), (64, 2048), (2048, 2047), (2080, 3), (4096, 2045), (32, 2049), (512, 2051), (544, 3000), (992, 2064),
     (1056, 2049), (1568, 4099), (2016, 2050), (2304, 3001), (3104, 2052), (1536, 14336), (1536, 12285), (4096, 28667),
-    (1024, 28672)])
+    (1024, 28672),
+    # where the form changes: 1024, 2048 and 4096 rows, 16, 32, 64 and 96 blocks a row, 2^16 in all
+    (512, 1024), (512, 4097), (480, 4369), (32, 65537), (544, 1024), (544, 1025), (1024, 4096), (1024, 4097), (1056, 1025), (2048, 2046),
+    (2080, 1024), (2080, 1027), (3072, 2048), (3104, 1025), (4096, 2047)])
 @pytest.mark.parametrize("rms", [True, False])
 def test_forms(rt, ora, n, rows, rms):
     r = np.random.default_rng(n + rows)
