@@ -261,10 +261,13 @@ hipError_t launch_qk_token(ATLAS_QK_PARAMS) {
 }
 
 // A token's units over several wavefronts, R register rows each, one
-// wavefront per workgroup.
+// wavefront per workgroup.  (Where one takes them all it is the token form,
+// without the division that finds a wavefront's token: 3.42 -> 3.34 us at
+// [1000, 1, 256].)
 template <int P, int HPR, int R, bool SEQ>
 hipError_t launch_qk_split(ATLAS_QK_PARAMS) {
     const uint32_t total = q_heads + has_key;
+    if (R < 9 && total <= R * HPR) return launch_qk_token<P, HPR, 1, SEQ>(ATLAS_QK_ARGS);
     const uint64_t waves = static_cast<uint64_t>(tokens) * ((total + R * HPR - 1) / (R * HPR));
     if (waves > 0x7fffffffu) return hipErrorInvalidValue;
     ATLAS_QK_LAUNCH(R, 1, true, static_cast<uint32_t>(waves))
@@ -285,9 +288,11 @@ hipError_t launch_qk_split(ATLAS_QK_PARAMS) {
 //             4352 (256 x 17) 4.44   4.47   4.61   5.35         10.8
 //             6912 (768 x 9)  6.10   5.23   5.23   5.73
 //             9000 (1000 x 9) 7.18   6.85   5.78   6.07
+//             10500 (700 x 15) 8.35  8.10   6.30   7.73
 //             13056 (768 x 17) 8.99  8.88   7.56   6.73         14.9
 //             34816 (2048 x 17) 19.2 16.8   16.0   13.5         22.9
 //   512       1152 (128 x 9)  4.48   5.07   5.32   5.93
+//             2048 (128 x 16) 5.44   5.71   6.07   8.15
 //             4352 (256 x 17) 7.75   6.29   6.34   7.59         12.8
 //             8704 (512 x 17) 11.8   10.4   9.05   8.81         16.8
 //   128       1152 (128 x 9)  2.96   3.03   3.30   3.91
@@ -300,16 +305,25 @@ hipError_t launch_qk_split(ATLAS_QK_PARAMS) {
 // its units ([2048, 4 + 1, 256] 6.09 us against 7.44 with four units each),
 // four tokens per workgroup ([4096, 8 + 1, 256] 14.17 us against 14.25-14.33
 // with one); the tree sum has no chain to spread, so it takes them from 768
-// tokens ([1000, 8 + 1, 256] 5.66 against 6.15).
+// tokens ([1000, 8 + 1, 256] 5.66 against 6.15).  So do tokens of few units
+// (to four at head_dim 128, to six wider) from 1200 tokens, which two or four
+// to a wavefront divide unevenly (5 as 4 + 1; us, R = 1 / 2 / 4 / token):
+//   head_dim 256  3 x 1500  5.13  5.09  4.88  4.74      5 x 1000  -     5.12  -     5.57
+//                 5 x 1500  6.75  5.94  6.15  5.75      5 x 2047  7.98  8.22  7.76  6.21
+//   head_dim 512  3 x 1250  7.31  6.84  6.32  6.20      3 x 1000  -     6.18  -     6.27
+//                 5 x 1500  11.3  10.1  8.93  8.03      5 x 1000  -     -     7.24  7.43
+//   head_dim 128  3 x 1750  4.48  4.42  4.04  3.99      6 x 1500  -     -     4.49  4.67
 template <int P, int HPR, bool SEQ>
 hipError_t launch_qk_p(ATLAS_QK_PARAMS) {
-    constexpr uint32_t kOne = P == 4 ? 1800 : (P == 2 ? 4500 : 2500);
+    constexpr uint32_t kOne = P == 4 ? 2100 : (P == 2 ? 4500 : 2500);
     constexpr uint32_t kTwo = P == 4 ? 5000 : (P == 2 ? 7000 : 10000);
     constexpr uint32_t kFour = P == 4 ? 8500 : (P == 2 ? 11000 : 20000);
+    constexpr uint32_t kFew = P == 1 ? 4 : 6;
     const uint32_t total = q_heads + has_key;
     const uint64_t units = static_cast<uint64_t>(tokens) * total;
     if (total <= 16 && tokens >= 2048) return launch_qk_token<P, HPR, 4, SEQ>(ATLAS_QK_ARGS);
     if (total <= 16 && tokens >= 768 && !SEQ) return launch_qk_token<P, HPR, 1, SEQ>(ATLAS_QK_ARGS);
+    if (HPR == 1 && total <= kFew && tokens >= 1200) return launch_qk_token<P, HPR, 1, SEQ>(ATLAS_QK_ARGS);
     if (units < kOne) return launch_qk_split<P, HPR, 1, SEQ>(ATLAS_QK_ARGS);
     if (units < kTwo) return launch_qk_split<P, HPR, 2, SEQ>(ATLAS_QK_ARGS);
     if (units < kFour) return launch_qk_split<P, HPR, 4, SEQ>(ATLAS_QK_ARGS);

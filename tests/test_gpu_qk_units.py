@@ -18,6 +18,10 @@ SHAPES = [
     (256, 32, True, 340), (256, 7, False, 1000), (256, 8, True, 1223),
     (512, 16, True, 5), (512, 16, True, 110), (512, 24, True, 210), (512, 16, True, 501), (512, 9, True, 850),
     (512, 33, True, 253),
+    # one wavefront with a token's few units, and the token count from which it takes up to four or six
+    (64, 2, False, 9), (64, 3, True, 1300), (128, 1, False, 5), (128, 1, True, 1200), (128, 5, True, 1207),
+    (256, 1, False, 1000), (256, 4, True, 1199), (256, 4, True, 1200), (256, 6, True, 1490), (512, 1, True, 1150),
+    (512, 2, True, 1201), (512, 15, True, 131), (512, 6, True, 1210),
 ]
 
 
