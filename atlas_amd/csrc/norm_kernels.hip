@@ -653,8 +653,8 @@ __global__ __launch_bounds__(RUN ? 64 * (kRunHelpers + 1) : 64) void rms_reg_ker
 }
 
 // Register-engine configuration, same bits each way.  Measured on MI355X:
-//  * rows < 2048 (to 512 wide: wider rows are the row-per-workgroup engine's,
-//    rms_row_engine): one row per wavefront, and past the first chunk the
+//  * rows < 2048 (to 512 wide, and to 800 rows from 384 wide: the others are
+//    the row-per-workgroup engine's, rms_row_engine): one row per wavefront, and past the first chunk the
 //    parallel fold as one run with its scans computed ahead by helper
 //    wavefronts (RUN; kRunHelpers): [1, 512] 2.7 us, [256, 512] 3.3;
 //  * rows >= 2048, plain RMSNorm: one row per wavefront, parallel fold

@@ -466,16 +466,23 @@ hipError_t launch_mode(hipStream_t s, const NormArgs& a, bool tree) {
 }  // namespace
 
 // Sequential order, us by the per-wavefront engine (with its helpers) / by
-// this one, residual: [1, 512] 2.7 / 2.7, [1, 768] 2.9 / 2.8, [1, 320] 2.5 / 2.7;
-// to 512 wide it takes over as rows queue: [700, 512] 3.9 / 4.0, [1000, 512]
-// 4.9 / 4.4, [700, 260] 3.9 / 4.4, [1000, 260] 5.0 / 4.8.  From 2048 rows up to
-// 2048 wide two rows a wavefront keep more loads in flight: [2048, 1536]
-// 9.8 / 9.9, [4096, 1536] 13.6 / 16.8 ([2047, 1536], one row a wavefront:
-// 14.5 / 9.9).  Past 2048 wide there is no other engine to 8192.
+// this one, residual epilogue:
+//   rows       1            64           256          512          1000         2047
+//   516 wide   3.06 / 3.12  4.08 / 4.04  4.29 / 4.20  4.56 / 4.57  6.56 / 5.33  10.5 / 7.94
+//   576        3.10 / 3.10  3.85 / 3.88  4.05 / 3.92  4.46 / 4.22  6.23 / 4.88  10.0 / 7.47
+//   768        3.16 / 3.11  3.97 / 3.81  4.19 / 4.04  4.50 / 4.44  6.52 / 5.32  10.4 / 7.86
+//   1000       3.66 / 3.30  4.44 / 4.08  4.74 / 4.44  5.12 / 4.95  7.37 / 5.76  11.3 / 8.45
+// To 512 wide it takes over as rows queue ([700, 512] 3.9 / 4.0, [1000, 512]
+// 5.27 / 4.82, [2047, 512] 7.58 / 7.22, [1000, 384] 5.02 / 4.70, [2047, 384]
+// 7.25 / 7.12), below 384 it does not pay ([1700, 260] 6.55 / 6.91, [1700, 320]
+// 6.29 / 6.55).  From 2048 rows up to 2048 wide two rows a wavefront keep more
+// loads in flight: [2048, 576] 6.7 (7.5 by this one at 2047), [2048, 1536]
+// 9.8 / 9.9, [4096, 1536] 13.6 / 16.8 (one row a wavefront: [2047, 1536] 14.5 / 9.9).  Past 2048 wide
+// there is no other engine to 8192.
 bool rms_row_engine(const NormArgs& a, bool tree) {
     if (a.hidden > 2048) return a.hidden <= 8192;
     if (tree || a.rows >= 2048) return false;
-    return a.hidden > 512 || (a.hidden > 256 && a.rows > 800);
+    return a.hidden > 512 || (a.hidden >= 384 && a.rows > 800);
 }
 
 hipError_t launch_rms_norm_row_f32(hipStream_t stream, NormMode mode, bool tree, const NormArgs& a) {

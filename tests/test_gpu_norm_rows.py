@@ -26,7 +26,7 @@ def test_exact_rows(rt, ora, hidden, mode):
 
 # rows past the eight-wavefront shapes', and the last and first of each engine
 ROWS = [(513, 1028), (512, 2048), (513, 2048), (513, 2052), (513, 3072), (513, 3076), (513, 4096), (768, 4100), (768, 6144),
-        (256, 8192), (257, 6148), (257, 8192), (1, 512), (1, 516), (800, 260), (801, 260), (800, 512), (801, 512),
+        (256, 8192), (257, 6148), (257, 8192), (1, 512), (1, 516), (800, 260), (801, 260), (801, 380), (800, 384), (801, 384), (2047, 380), (800, 512), (801, 512),
         (2047, 516), (2047, 1536), (2047, 2048), (2048, 516), (2048, 2048)]
 
 
