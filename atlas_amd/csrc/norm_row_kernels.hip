@@ -485,14 +485,29 @@ bool rms_row_engine(const NormArgs& a, bool tree) {
     return a.hidden > 512 || (a.hidden >= 384 && a.rows > 800);
 }
 
-hipError_t launch_rms_norm_row_f32(hipStream_t stream, NormMode mode, bool tree, const NormArgs& a) {
-    switch (mode) {
-        case kNormPlain: return launch_mode<kNormPlain>(stream, a, tree);
-        case kNormResidual: return launch_mode<kNormResidual>(stream, a, tree);
-        case kNormAddNorm: return launch_mode<kNormAddNorm>(stream, a, tree);
-        case kNormAddScale: return launch_mode<kNormAddScale>(stream, a, tree);
+hipError_t launch_rms_norm_row_f32(hipStream_t stream, NormMode mode, bool tree, const NormArgs& args) {
+    // a launch's threads are counted in 32 bits (past that only the remainder
+    // runs, without an error), and a row here has up to 512
+    constexpr uint32_t kRowsPerLaunch = 0xffffffffu / 512;
+    hipError_t e = hipErrorInvalidValue;
+    for (uint64_t r0 = 0; r0 < args.rows; r0 += kRowsPerLaunch) {
+        const uint64_t at = r0 * args.hidden, left = args.rows - r0;
+        NormArgs a = args;
+        a.rows = static_cast<uint32_t>(left < kRowsPerLaunch ? left : kRowsPerLaunch);
+        a.x += at;
+        a.out += at;
+        if (a.residual) a.residual += at;
+        if (a.normalized) a.normalized += at;
+        if (a.residual_out) a.residual_out += at;
+        switch (mode) {
+            case kNormPlain: e = launch_mode<kNormPlain>(stream, a, tree); break;
+            case kNormResidual: e = launch_mode<kNormResidual>(stream, a, tree); break;
+            case kNormAddNorm: e = launch_mode<kNormAddNorm>(stream, a, tree); break;
+            case kNormAddScale: e = launch_mode<kNormAddScale>(stream, a, tree); break;
+        }
+        if (e != hipSuccess) return e;
     }
-    return hipErrorInvalidValue;
+    return e;
 }
 
 }  // namespace atlas

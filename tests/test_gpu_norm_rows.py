@@ -86,3 +86,36 @@ def test_in_place(rt, ora):
     rt.rms_norm_residual(work, w, state, work, state, rows, h, eps)
     rt.sync()
     assert_bits("aliased", [work.download(rows * h), state.download(rows * h)], [np.asarray(n_exp), np.asarray(out_exp)])
+
+
+def test_more_rows_than_one_launch(rt, ora):
+    """A launch holds fewer than 2^32 threads, 512 a row at this width; the rows
+    around 2^23 (137 GB of them, in place) in both orders."""
+    from atlas_amd import ATLAS_REDUCTION_SEQUENTIAL, ATLAS_REDUCTION_WIDE, OperatorError
+
+    hidden, rows, eps = 4100, (1 << 23) + 3, 1e-6
+    try:
+        buf = rt.alloc(4 * hidden * rows)
+    except OperatorError as e:
+        assert e.kind == "OutOfMemory"
+        pytest.skip("needs 137 GB of free device memory")
+    try:
+        rng = np.random.default_rng(1)
+        w = rng.standard_normal(hidden).astype(np.float32)
+        dw = rt.upload(w)
+        near = [0, (1 << 23) - 2, (1 << 23) - 1, 1 << 23, rows - 1]
+        for order in (ATLAS_REDUCTION_SEQUENTIAL, ATLAS_REDUCTION_WIDE):
+            x = rng.standard_normal((len(near), hidden)).astype(np.float32)
+            for r, v in zip(near, x):
+                buf.offset(4 * hidden * r).upload(v)
+            rt.set_reduction(order)
+            rt.rms_norm(buf, dw, buf, rows, hidden, eps)
+            rt.sync()
+            got = np.stack([buf.offset(4 * hidden * r).download(hidden) for r in near])
+            exp = np.asarray(ora.rms_norm(x.reshape(-1), w, len(near), hidden, eps)).reshape(got.shape)
+            # 4100 squares summed in another order: at most 4100 x 2^-24 of the sum, half of it of its scale
+            assert np.array_equal(got, exp) if order == ATLAS_REDUCTION_SEQUENTIAL else \
+                np.max(np.abs(got - exp) / np.abs(exp)) <= 2 * 4100 * 2.0 ** -24
+    finally:
+        rt.set_reduction(ATLAS_REDUCTION_SEQUENTIAL)
+        rt.free(buf)
