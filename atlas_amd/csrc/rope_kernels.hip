@@ -268,9 +268,7 @@ template <int P, int HPR, int R, bool SEQ>
 hipError_t launch_qk_split(ATLAS_QK_PARAMS) {
     const uint32_t total = q_heads + has_key;
     if (R < 9 && total <= R * HPR) return launch_qk_token<P, HPR, 1, SEQ>(ATLAS_QK_ARGS);
-    const uint64_t waves = static_cast<uint64_t>(tokens) * ((total + R * HPR - 1) / (R * HPR));
-    if (waves > 0x7fffffffu) return hipErrorInvalidValue;
-    ATLAS_QK_LAUNCH(R, 1, true, static_cast<uint32_t>(waves))
+    ATLAS_QK_LAUNCH(R, 1, true, tokens * ((total + R * HPR - 1) / (R * HPR)))
 }
 
 // Units per wavefront by the launch's units (tokens x heads).  A wavefront
@@ -319,7 +317,26 @@ hipError_t launch_qk_p(ATLAS_QK_PARAMS) {
     constexpr uint32_t kTwo = P == 4 ? 5000 : (P == 2 ? 7000 : 10000);
     constexpr uint32_t kFour = P == 4 ? 8500 : (P == 2 ? 11000 : 20000);
     constexpr uint32_t kFew = P == 1 ? 4 : 6;
+    constexpr uint32_t D = 128 * P / HPR;
     const uint32_t total = q_heads + has_key;
+    // a launch's threads are counted in 32 bits: at most 2^26 wavefronts, one
+    // per token or, past 16 units, one per 9 register rows
+    const uint32_t parts = total > 16 ? (total + 9 * HPR - 1) / (9 * HPR) : 1u;
+    const uint32_t most = ((1u << 26) - 8) / parts;
+    for (; tokens > most; tokens -= most) {
+        const hipError_t e = launch_qk_p<P, HPR, SEQ>(stream, q, k, qw, kw, c, sn, qo, ko, most, q_heads, has_key, rope_stride, eps);
+        if (e != hipSuccess) return e;
+        if (q_heads) {
+            q += static_cast<size_t>(most) * q_heads * D;
+            qo += static_cast<size_t>(most) * q_heads * D;
+        }
+        if (has_key) {
+            k += static_cast<size_t>(most) * D;
+            ko += static_cast<size_t>(most) * D;
+        }
+        c += static_cast<size_t>(most) * rope_stride;
+        sn += static_cast<size_t>(most) * rope_stride;
+    }
     const uint64_t units = static_cast<uint64_t>(tokens) * total;
     if (total <= 16 && tokens >= 2048) return launch_qk_token<P, HPR, 4, SEQ>(ATLAS_QK_ARGS);
     if (total <= 16 && tokens >= 768 && !SEQ) return launch_qk_token<P, HPR, 1, SEQ>(ATLAS_QK_ARGS);

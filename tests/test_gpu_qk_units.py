@@ -46,3 +46,42 @@ def test_units_tree_sum(rt, ora, head_dim, q_heads, tokens):
     # relative change of a row's sum, half of it that of its scale
     for g, e in zip(got, cases.qk_oracle(ora, inp, m)):
         assert np.linalg.norm(g - e) <= 1e-6 * np.linalg.norm(e)
+
+
+def test_more_tokens_than_one_launch(rt, ora):
+    """A launch holds fewer than 2^26 wavefronts and 18 + 1 heads take two a
+    token: the tokens around 2^25 (165 GB of heads, in place)."""
+    from atlas_amd import OperatorError
+
+    d, qh, half = 64, 18, 32
+    tokens, split = (1 << 25) + 5, ((1 << 26) - 8) // 2
+    bufs = []
+    try:
+        for n in (tokens * qh * d, tokens * d, tokens * half):
+            bufs.append(rt.alloc(4 * n))
+    except OperatorError as e:
+        assert e.kind == "OutOfMemory"
+        for b in bufs:
+            rt.free(b)
+        pytest.skip("needs 168 GB of free device memory")
+    q, k, rope = bufs  # cosine and sine share their rows
+    try:
+        rng = np.random.default_rng(2)
+        near = np.array([0, split - 1, split, (1 << 25) - 1, 1 << 25, tokens - 1])
+        x = rng.standard_normal((near.size, qh * d), dtype=np.float32)
+        y = rng.standard_normal((near.size, d), dtype=np.float32)
+        cs = rng.standard_normal((near.size, half), dtype=np.float32)
+        w = rng.standard_normal((2, d), dtype=np.float32)
+        for i, t in enumerate(near):
+            for b, v in ((q, x[i]), (k, y[i]), (rope, cs[i])):
+                b.offset(v.nbytes * int(t)).upload(v)
+        qw, kw = rt.upload(w[0]), rt.upload(w[1])
+        rt.qk_norm_rope(q, k, qw, kw, rope, rope, q, k, tokens, qh, 1, d, half, 1e-6)
+        rt.sync()
+        eq, ek = ora.qk_norm_rope(x, y, w[0], w[1], cs, cs, near.size, qh, True, d, half, 1e-6)
+        for i, t in enumerate(near):
+            assert np.array_equal(q.offset(4 * qh * d * int(t)).download(qh * d), eq.reshape(x.shape)[i]), t
+            assert np.array_equal(k.offset(4 * d * int(t)).download(d), ek.reshape(y.shape)[i]), t
+    finally:
+        for b in bufs:
+            rt.free(b)
