@@ -9,7 +9,6 @@
 
 #include <hip/hip_runtime.h>
 
-#include <atomic>
 #include <chrono>
 #include <cmath>
 #include <cstdarg>
@@ -34,12 +33,13 @@ struct atlas_hip_ctx {
     // no-allocation soft cap + argmax entry point); resolved at init
     void* argmax_scratch = nullptr;
     // buffers of the host-slice ops (Scratch): one pinned, one on the device,
-    // of the same layout; idle between calls, which all end synchronized
+    // of the same layout; idle between calls, which all end synchronized and
+    // take turns (HostCall)
+    std::mutex host_ops;
     uint8_t* host_ops_pinned = nullptr;
     uint8_t* host_ops_device = nullptr;
     size_t host_ops_bytes = 0;
     hipEvent_t host_ops_event[2] = {};
-    std::atomic<bool> host_ops_busy{false};
     std::string last_error;
     atlas_hip_telemetry tel{};
 };
@@ -969,6 +969,18 @@ namespace {
 constexpr size_t kHostOpsMax = size_t{16} << 20;
 constexpr size_t kHostOpsMin = size_t{1} << 20;
 
+// A host-slice call on a context: threads that share one take turns, so the kept
+// buffers, the telemetry and the error text are one call's at a time.
+struct HostCall {
+    std::unique_lock<std::mutex> turn;
+    int rc = ATLAS_ERR_INVALID_INPUT;
+    explicit HostCall(atlas_hip_ctx* ctx) {
+        if (!ctx) return;
+        turn = std::unique_lock<std::mutex>(ctx->host_ops);
+        rc = enter(ctx);
+    }
+};
+
 // Makes the context's buffers hold `bytes` (at most kHostOpsMax); false: the call
 // allocates its own.
 bool reserve_host_ops(atlas_hip_ctx* ctx, size_t bytes) {
@@ -996,8 +1008,8 @@ bool reserve_host_ops(atlas_hip_ctx* ctx, size_t bytes) {
 //
 // A call that fits is served from the context's buffers: the inputs are copied
 // to pinned memory side by side and go up in one transfer, the output comes
-// down in one, and the host waits once.  A call that finds the buffers taken by
-// another thread's allocates its own.  Against a buffer for each operand with
+// down in one, and the host waits once.  Telemetry counts its operands as if
+// each had been allocated, the kept buffers not at all.  Against a buffer for each operand with
 // a transfer from the caller's pageable memory and a wait each, us a call: silu
 // of 256 bytes 53 -> 30, of 295 KB 62 -> 48, of 2.1 MB 304 -> 203, add of 4.2 MB
 // 660 -> 490; RMSNorm and RoPE of [128, 576] 77 and 90 -> 50.  Sending an input
@@ -1012,15 +1024,10 @@ public:
             fits = fits && bytes <= kHostOpsMax;
             total += fits ? padded(bytes) : 0;
         }
-        if (!fits || total > kHostOpsMax || c->host_ops_busy.exchange(true)) return;
-        pooled_ = reserve_host_ops(c, total);
-        if (!pooled_) c->host_ops_busy = false;
+        pooled_ = fits && total <= kHostOpsMax && reserve_host_ops(c, total);
     }
     ~Scratch() {
-        if (pooled_) {
-            ctx_->tel.resident_bytes -= taken_;
-            ctx_->host_ops_busy = false;
-        }
+        if (pooled_) ctx_->tel.resident_bytes -= taken_;
         for (int i = 0; i < n_; ++i) atlas_hip_free(ctx_, ptrs_[i]);
     }
     Scratch(const Scratch&) = delete;
@@ -1146,7 +1153,8 @@ int atlas_ops_embedding(atlas_hip_ctx* ctx, const float* table, size_t table_len
                         const uint32_t* token_ids, size_t token_count, float* output, size_t output_len,
                         atlas_dispatch_timing* timing) {
     const auto t0 = std::chrono::steady_clock::now();
-    int rc = enter(ctx);
+    const HostCall call(ctx);
+    int rc = call.rc;
     if (rc) return rc;
     size_t table_elems = 0, total = 0;
     if (!mul_ok(vocabulary, hidden, &table_elems) || table_len != table_elems)
@@ -1174,7 +1182,8 @@ int atlas_ops_embedding_q6_k(atlas_hip_ctx* ctx, const uint8_t* weights, size_t 
                              size_t hidden, const uint32_t* token_ids, size_t token_count, float* output,
                              size_t output_len, atlas_dispatch_timing* timing) {
     const auto t0 = std::chrono::steady_clock::now();
-    int rc = enter(ctx);
+    const HostCall call(ctx);
+    int rc = call.rc;
     if (rc) return rc;
     if (hidden == 0 || hidden % 256 != 0 || token_count == 0 || !token_ids)
         return invalid(ctx, "Q6_K embedding dimensions or token IDs are invalid");
@@ -1203,7 +1212,8 @@ int atlas_ops_embedding_q6_k(atlas_hip_ctx* ctx, const uint8_t* weights, size_t 
 static int binary_op(atlas_hip_ctx* ctx, int op, const float* lhs, size_t lhs_len, const float* rhs, size_t rhs_len,
                      float* output, size_t output_len, atlas_dispatch_timing* timing) {
     const auto t0 = std::chrono::steady_clock::now();
-    int rc = enter(ctx);
+    const HostCall call(ctx);
+    int rc = call.rc;
     if (rc) return rc;
     if (lhs_len != rhs_len) return invalid(ctx, op == 0 ? "vector lengths differ" : "multiply requires equally sized non-empty vectors");
     if (op == 1 && lhs_len == 0) return invalid(ctx, "multiply requires equally sized non-empty vectors");
@@ -1240,7 +1250,8 @@ int atlas_ops_multiply(atlas_hip_ctx* ctx, const float* lhs, size_t lhs_len, con
 static int unary_op(atlas_hip_ctx* ctx, int op, const float* input, size_t input_len, float scalar, float* output,
                     size_t output_len, atlas_dispatch_timing* timing) {
     const auto t0 = std::chrono::steady_clock::now();
-    int rc = enter(ctx);
+    const HostCall call(ctx);
+    int rc = call.rc;
     if (rc) return rc;
     if (!fits_u32(input_len)) return invalid(ctx, "input is too large");
     if (output_len != input_len || (input_len && (!input || !output))) return invalid(ctx, "output has the wrong length");
@@ -1280,7 +1291,8 @@ int atlas_ops_rms_norm(atlas_hip_ctx* ctx, const float* input, size_t input_len,
                        const float* weight, size_t weight_len, float epsilon, float* output, size_t output_len,
                        atlas_dispatch_timing* timing) {
     const auto t0 = std::chrono::steady_clock::now();
-    int rc = enter(ctx);
+    const HostCall call(ctx);
+    int rc = call.rc;
     if (rc) return rc;
     size_t elements = 0;
     if (!mul_ok(rows, hidden, &elements)) return invalid(ctx, "RMSNorm dimensions overflow");
@@ -1305,7 +1317,8 @@ int atlas_ops_rope(atlas_hip_ctx* ctx, const float* input, size_t input_len, siz
                    const float* cosine, size_t cosine_len, const float* sine, size_t sine_len, float* output,
                    size_t output_len, atlas_dispatch_timing* timing) {
     const auto t0 = std::chrono::steady_clock::now();
-    int rc = enter(ctx);
+    const HostCall call(ctx);
+    int rc = call.rc;
     if (rc) return rc;
     size_t elements = 0;
     if (!mul_ok(rows, hidden, &elements)) return invalid(ctx, "RoPE input overflow");

@@ -36,6 +36,8 @@
  *    epilogues, QK-norm + RoPE, the stable group norm), so those stay
  *    bit-identical to the CPU operators.
  *  - One context per host thread; calls on one context are not re-entrant.
+ *    The atlas_ops_* ops alone may be called on one context from several
+ *    threads: they take turns.
  */
 #ifndef ATLAS_HIP_OPS_H
 #define ATLAS_HIP_OPS_H
@@ -71,7 +73,11 @@ typedef struct atlas_dispatch_timing {
 } atlas_dispatch_timing;
 
 /* RuntimeTelemetry (crates/atlas-metal/src/lib.rs:91-193), the subset that
- * applies to this library. */
+ * applies to this library.  An atlas_ops_* op counts each operand as one
+ * allocation, resident while it runs.  Not counted: the buffers that serve
+ * operands of at most 16 MiB in all, which a context keeps from one such op to
+ * the next and frees when it is destroyed (at most 16 MiB of device and 16 MiB
+ * of pinned host memory, grown by doubling from 1 MiB). */
 typedef struct atlas_hip_telemetry {
     uint64_t dispatches;
     uint64_t syncs;

@@ -76,11 +76,13 @@ def test_telemetry_and_refusals():
     assert np.array_equal(ops.add(x, x)[0], x + x)
 
 
-def test_threads_on_one_context(ops):
-    """Calls that overlap take the kept buffers one at a time and allocate
-    otherwise: each gets its own result."""
+def test_threads_on_one_context():
+    """Threads that share a context take turns, in the kept buffers and past
+    them: each call gets its own result, and the telemetry of all of them adds up."""
+    ops = NeuralOps()
     rng = np.random.default_rng(9)
-    inputs = [rng.standard_normal(n, dtype=np.float32) for n in (1000, 70001, 300000, 64)]
+    inputs = [rng.standard_normal(n, dtype=np.float32) for n in (1000, 70001, 300000, 64, KEPT // 4, 2)]
+    before = ops.rt.telemetry()
     wrong = []
 
     def work(x):
@@ -95,3 +97,12 @@ def test_threads_on_one_context(ops):
     for t in threads:
         t.join()
     assert wrong == []
+    after = ops.rt.telemetry()
+    calls, values = 20 * len(inputs), 20 * sum(x.size for x in inputs)
+    assert after.allocations - before.allocations == 3 * calls
+    assert after.dispatches - before.dispatches == calls
+    assert after.upload_bytes - before.upload_bytes == 8 * values
+    assert after.readback_bytes - before.readback_bytes == 4 * values
+    assert after.resident_bytes == before.resident_bytes
+    # one call at a time: the largest one's operands, not several calls'
+    assert after.peak_resident_bytes == before.resident_bytes + 3 * KEPT
