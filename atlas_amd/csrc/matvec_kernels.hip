@@ -23,21 +23,26 @@
 // 4-bit codes costs more VALU work (a conversion and an FMA per weight) than
 // its bytes take to arrive, so the codes meet the input on the matrix cores as
 // integers (v_mfma_i32_4x4x4_16b_i8: 16 independent 4 x 4 x 4 products):
-//  * each 32-value block of y = x * w becomes 31-bit fixed point under the
-//    block's largest |y| (relative 2^-31; f32 itself holds 2^-24) and is split
-//    into four signed byte digits; the digits of four consecutive values are
-//    one word per digit, the A operand's four rows;
+//  * each 32-value block of y = x * w becomes fixed point, rounded to steps of
+//    2^-30 of the power of two above the block's largest |y| (values below about
+//    2^-6 of that power lose bits to it, at most half a step each), and is split
+//    into four signed byte digits; the digits of four consecutive values are one
+//    word per digit, the A operand's four rows;
 //  * a lane holds one weight row's block as loaded, 16 (q - 8) in the bytes of
 //    eight words by a mask and a shift (q ^ 8 in a byte's high nibble is
 //    16 (q - 8) in two's complement), the B operand's columns: lane l is row
 //    l % 4 of the wavefront's four and block l / 4 of the pass's sixteen;
 //  * eight products accumulate a block exactly in i32, one register per digit
-//    and in the lane of its row; the digits meet in two 24-bit halves, one f32
-//    fma, and the block's scale d goes on with the row's running sum.
+//    and in the lane of its row; the digits meet in two halves of up to 28
+//    bits, rounded as they become f32, and one fma, and the block's scale d goes
+//    on with the row's running sum.
 // ~45 VALU operations a block instead of ~85, 32 bytes of the input read from
-// LDS per lane and block instead of 128, and a dot whose only roundings are
-// three per block: the error against float64 falls from 3e-8 to 9e-9 of the
-// sum of magnitudes.
+// LDS per lane and block instead of 128.  Against float64, of the sum of
+// |products| (root mean square over [2600, 1536]): 3.0e-9 on N(0, 1) inputs
+// (vector dot 1.1e-8), 1.2e-8 with a value of 1000 in each block (3.7e-8), and
+// 1.2e-8 where that value meets code 8, so that its step is all it leaves
+// (vector dot, which takes the offset 8 of the whole block, 1.0e-6; the steps
+// truncated instead of rounded 2.3e-8).
 #include "device_common.hpp"
 #include "launch.hpp"
 
@@ -77,12 +82,12 @@ __device__ __forceinline__ float sum_of_row(float v) {
 }
 
 // Four values as signed byte digits: word p holds digit p (weight 256^p) of
-// the four, after scaling by 2^shift (|v 2^shift| <= 2^30).
+// the four, scaled by 2^shift and rounded (|v 2^shift| < 2^30).
 __device__ __forceinline__ void digit_words(const f32x4 v, int shift, uint32_t (&word)[4]) {
     uint32_t t[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        const int q = static_cast<int>(__builtin_ldexpf(v[i], shift));
+        const int q = static_cast<int>(__builtin_rintf(__builtin_ldexpf(v[i], shift)));
         // a digit d in [-128, 127] is the byte d + 128 of q + 0x808080 (the
         // top one has no bias), so clearing the bias leaves two's complement
         t[i] = (static_cast<uint32_t>(q) + 0x00808080u) ^ 0x00808080u;
@@ -326,7 +331,7 @@ hipError_t launch_shape(hipStream_t stream, MatvecArgs a, uint32_t groups) {
 
 // Groups of four rows per wavefront: the input's digits cost a workgroup about
 // as much as one group, so the most that leave the card some 448 workgroups
-// whose last round over the CUs is at least nine tenths full.
+// which fill their rounds over the CUs to nine tenths on average.
 uint32_t staged_groups(uint32_t rows) {
     for (uint32_t groups : {4u, 2u}) {
         const uint32_t blocks = (rows + 16 * groups - 1) / (16 * groups), rounds = (blocks + 255) / 256;
