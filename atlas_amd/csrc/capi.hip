@@ -759,7 +759,7 @@ static int q4_matvec(atlas_hip_ctx* ctx, const float* input, const float* rms_we
     a.rms_weight = rms_weight;
     a.epsilon = epsilon;
     a.input_width = input_width;
-    a.segments = segments;
+    a.segments = static_cast<uint16_t>(segments);
     a.ple = ple;
     a.ple_offset = ple_offset;
     for (uint32_t i = 0; i < segments; ++i) {

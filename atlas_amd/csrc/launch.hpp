@@ -122,12 +122,19 @@ struct MatvecArgs {
     uint32_t ple_offset;
     float epsilon;
     uint32_t input_width;  // multiple of 32, <= q4_0_matvec_max_input()
-    uint32_t segments;     // 1..3
+    uint16_t segments;     // 1..3
+    uint16_t groups;       // of four rows per wavefront; filled by the launcher
     const uint8_t* weights[3];
     float* output[3];
     uint32_t width[3];
     uint32_t tile_begin[3];  // filled by the launcher
 };
+// All of a kernel's arguments in at most 112 bytes: past that, launches issued
+// one by one cost the host 0.4 us more in most processes (104 and 112 bytes 3.6
+// us a launch, 116 to 192 4.0-4.2, in the others 3.1 at any size), and the kernel
+// up to 0.45 us (gate/up at 1536: 4.65 and 5.1).  Launches of a graph do not
+// differ.
+static_assert(sizeof(MatvecArgs) == 112, "kernel argument bytes");
 uint32_t q4_0_matvec_max_input();
 hipError_t launch_q4_0_matvec(hipStream_t stream, MatvecArgs a);
 

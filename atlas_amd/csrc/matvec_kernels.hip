@@ -129,7 +129,7 @@ __host__ __device__ constexpr uint32_t stage_bytes(int nbt) { return 4 * 16 * 18
 // unit takes ~225 cycles a pass over; KS wavefronts share a group's rows, NBT
 // passes each.
 template <int NBT, int KS, bool STAGED>
-__global__ __launch_bounds__(256) void q4_0_matvec_kernel(MatvecArgs a, uint32_t groups) {
+__global__ __launch_bounds__(256) void q4_0_matvec_kernel(MatvecArgs a) {
     static_assert(!STAGED || KS == 1, "a staged row belongs to one wavefront");
     constexpr int kJ = (NBT * KS * kPassBlocks * 32 / 4 + 255) / 256;  // float4 of x per thread
     constexpr int kLoads = STAGED ? (4 * 18 * NBT + 63) / 64 : NBT;  // 16-byte loads per lane and group
@@ -138,6 +138,7 @@ __global__ __launch_bounds__(256) void q4_0_matvec_kernel(MatvecArgs a, uint32_t
     const uint32_t tid = threadIdx.x, lane = tid % kWave;
     const uint32_t wave = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(tid / kWave));
     const uint32_t n = a.input_width, n4 = n / 4, nb = n / 32, row_bytes = nb * kQ4Block;
+    const uint32_t groups = a.groups;
     const uint32_t rows = kPassRows * groups * kWaves / KS;  // rows per workgroup
 
     // The projection this workgroup's rows belong to (segments are tile ranges).
@@ -318,6 +319,7 @@ __global__ __launch_bounds__(256) void q4_0_matvec_kernel(MatvecArgs a, uint32_t
 
 template <int NBT, int KS, bool STAGED>
 hipError_t launch_shape(hipStream_t stream, MatvecArgs a, uint32_t groups) {
+    a.groups = static_cast<uint16_t>(groups);
     const uint32_t rows = kPassRows * groups * kWaves / KS;
     uint32_t tiles = 0;
     for (uint32_t i = 0; i < a.segments; ++i) {
@@ -325,7 +327,7 @@ hipError_t launch_shape(hipStream_t stream, MatvecArgs a, uint32_t groups) {
         tiles += (a.width[i] + rows - 1) / rows;
     }
     const size_t lds = plane_bytes(a.input_width / 32) + (STAGED ? kWaves * stage_bytes(NBT) : 0);
-    hipLaunchKernelGGL((q4_0_matvec_kernel<NBT, KS, STAGED>), dim3(tiles), dim3(kWaves * kWave), lds, stream, a, groups);
+    hipLaunchKernelGGL((q4_0_matvec_kernel<NBT, KS, STAGED>), dim3(tiles), dim3(kWaves * kWave), lds, stream, a);
     return hipGetLastError();
 }
 
