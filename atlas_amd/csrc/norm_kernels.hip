@@ -382,10 +382,10 @@ struct FoldScansLds {
     uint32_t e0;
 };
 
-// RUN: helper wavefronts, one binade's scans each.  Measured on MI355X (C5
-// epilogues, with the head folded by candidate segments): four helpers
-// 4.54-4.56 us at 256 rows and 3.28-3.39 at one row, against 4.61-4.65 and
-// 3.37-3.50 with two helpers of two binades each.
+// RUN: helper wavefronts, one binade's scans each.  Measured on MI355X (residual
+// epilogue, with the head folded by candidate segments), four helpers / two of
+// two binades each: [1, 512] 2.59 / 2.60 us, [256, 320] 3.36 / 3.33, [700, 512]
+// 3.94 / 4.00; [2000, 260] 7.1 / 5.2, where the wavefronts queue.
 constexpr int kRunHelpers = 4;
 
 template <int R, int J, int MODE, bool PAR, bool STAGE, bool RUN>
@@ -397,16 +397,15 @@ __global__ __launch_bounds__(RUN ? 64 * (kRunHelpers + 1) : 64) void rms_reg_ker
     // compiler can wait for chunk j's loads alone before folding it.
     extern __shared__ f32x4 sq4[];
     constexpr bool kOperand = MODE != kNormPlain;
-    // RUN: one row; kRunHelpers more wavefronts compute the continuation's
-    // scans (fold_scan_ahead, one binade each) while the first folds the
-    // head (head_fold_candidates)
-    constexpr bool kRun = RUN && PAR && J > 1 && R == 1;
-    constexpr int kRunS = 4 * (J > 1 ? J - 1 : 1);
+    // RUN: one row of two chunks; kRunHelpers more wavefronts compute the
+    // second chunk's scans (fold_scan_ahead, one binade each) while the first
+    // folds the head (head_fold_candidates)
+    static_assert(!RUN || (PAR && !STAGE && R == 1 && J == 2), "the run is the second of two chunks");
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t h = a.hidden;
     const uint32_t nv = h >> 2;
     // RUN: a row's squares at their columns, zero-padded to 64 * J float4
-    const uint32_t stride4 = kRun ? 64u * J + 1 : nv + 1;
+    const uint32_t stride4 = RUN ? 64u * J + 1 : nv + 1;
     // the wavefront's R consecutive rows; the valid ones are r < nrows
     const uint32_t row0 = blockIdx.x * R;
     const uint32_t nrows = min(static_cast<uint32_t>(R), a.rows - row0);
@@ -415,39 +414,31 @@ __global__ __launch_bounds__(RUN ? 64 * (kRunHelpers + 1) : 64) void rms_reg_ker
     FoldScansLds<4>* scans_lds = reinterpret_cast<FoldScansLds<4>*>(sq4 + stride4);
     // RUN: chunk 0's squares again, laid out for head_fold_candidates
     f32x4* head_pad = sq4 + stride4 + (sizeof(FoldScansLds<4>) + 15) / 16;
-    // lane l's run: the 4 * (J - 1) consecutive squares from float4 64 + (J - 1) * l
-    auto read_run = [&](float (&run)[kRunS]) {
-#pragma unroll
-        for (int i = 0; i < J - 1; ++i) {
-            const f32x4 q = sq4[64u + (J - 1) * lane + i];
-            run[4 * i] = q.x;
-            run[4 * i + 1] = q.y;
-            run[4 * i + 2] = q.z;
-            run[4 * i + 3] = q.w;
-        }
+    // lane l's run: the 4 squares of float4 64 + l
+    auto read_run = [&](float (&run)[4]) {
+        const f32x4 q = sq4[64u + lane];
+        run[0] = q.x;
+        run[1] = q.y;
+        run[2] = q.z;
+        run[3] = q.w;
     };
-    if constexpr (kRun) {
+    if constexpr (RUN) {
         if (threadIdx.x >= 64) {  // the helper wavefronts
-            constexpr int kBph = 4 / kRunHelpers;
-            const uint32_t b0 = kBph * (static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) - 1u);
+            const uint32_t b = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) - 1u;
             __syncthreads();  // every square staged
             const f32x4 h0 = sq4[lane];
             const float approx = wave_sum_any_order_f32((h0.x + h0.y) + (h0.z + h0.w));
             // any-order and in-order sums of 256 squares differ by < 3e-5
             // relative, so this is a lower bound of the head's exponent
             const uint32_t e0 = __float_as_uint(approx * 0.999f) >> 23;
-            float run[kRunS];
+            float run[4];
             read_run(run);
-            const FoldScans<kBph> f = fold_scan_ahead<kRunS, kBph>(run, e0 + b0);
-#pragma unroll
-            for (int b = 0; b < kBph; ++b) {
-                scans_lds->inc[b0 + b][lane] = f.inc[b];
-                scans_lds->incl[b0 + b][lane] = f.incl[b];
-            }
+            const FoldScans<1> f = fold_scan_ahead<4, 1>(run, e0 + b);
+            scans_lds->inc[b][lane] = f.inc[0];
+            scans_lds->incl[b][lane] = f.incl[0];
             if (lane == 0) {
-#pragma unroll
-                for (int b = 0; b < kBph; ++b) scans_lds->bad[b0 + b] = f.bad[b];
-                if (b0 == 0) scans_lds->e0 = e0;
+                scans_lds->bad[b] = f.bad[0];
+                if (b == 0) scans_lds->e0 = e0;
             }
             __syncthreads();  // scans published
             return;
@@ -514,8 +505,8 @@ __global__ __launch_bounds__(RUN ? 64 * (kRunHelpers + 1) : 64) void rms_reg_ker
             }
             if (!par_chunk) {
                 sq4[r * stride4 + c] = f32x4{v.x * v.x, v.y * v.y, v.z * v.z, v.w * v.w};
-                if (kRun && j == 0) head_pad[lane + lane / 16] = f32x4{v.x * v.x, v.y * v.y, v.z * v.z, v.w * v.w};
-            } else if (kRun) {
+                if (RUN && j == 0) head_pad[lane + lane / 16] = f32x4{v.x * v.x, v.y * v.y, v.z * v.z, v.w * v.w};
+            } else if (RUN) {
                 // staged for the one-step continuation below (+0 past the row
                 // width: adding +0 leaves a sum of squares unchanged)
                 sq4[r * stride4 + creal] = creal < nv ? f32x4{v.x * v.x, v.y * v.y, v.z * v.z, v.w * v.w}
@@ -530,7 +521,7 @@ __global__ __launch_bounds__(RUN ? 64 * (kRunHelpers + 1) : 64) void rms_reg_ker
                 sqr[r][3] = in_row ? v.w * v.w : 0.0f;
             }
         }
-        if (par_chunk && !kRun) {
+        if (par_chunk && !RUN) {
             // two rows' scans side by side, else row by row (measured on
             // MI355X, residual at [4096, 1536]: 13.50-13.52 against
             // 13.63-13.65 us row by row; the inverse RMS likewise one chain
@@ -543,24 +534,24 @@ __global__ __launch_bounds__(RUN ? 64 * (kRunHelpers + 1) : 64) void rms_reg_ker
                     if (static_cast<uint32_t>(r) < nrows) sb[r] = fold_chunk_exact<4>(sqr[r], sb[r]);
             }
         }
-        if (!par_chunk && !kRun) {
+        if (!par_chunk && !RUN) {
             __syncthreads();
             if (lane < nrows)
                 s = fold_lds_chunk(sq4 + lane * stride4 + 64u * j, min(nv, 64u * (j + 1)) - 64u * j, s);
         }
-        if ((PAR && !kRun && j == 0) || (kTail && j == J - kTailN - 1)) {
+        if ((PAR && !RUN && j == 0) || (kTail && j == J - kTailN - 1)) {
             // the first chunk, where the sum crosses many binades and ties are
             // frequent, folds in order; broadcast each row's partial sum
 #pragma unroll
             for (int r = 0; r < R; ++r) sb[r] = readlane_u32(__float_as_uint(s), static_cast<uint32_t>(r));
         }
     }
-    if constexpr (kRun) {
+    if constexpr (RUN) {
         // The continuation (columns 256 .. 256 * J) as one run.  The helper
         // wavefronts compute its scans for four binades from a lower bound
         // of the head's exponent while this one folds the head (four
-        // segments folded from candidate starts and chained by selection,
-        // 5.13 -> 4.61 us per C5 epilogue at 256 rows with two helpers);
+        // segments folded from candidate starts and chained by selection:
+        // [1, 512] 2.59 us against 2.82 folded in order, [700, 512] 3.94 against 4.18);
         // the walk then has only the fold's real events (binade crossings,
         // ties) left.
         __syncthreads();  // every square staged
@@ -578,9 +569,9 @@ __global__ __launch_bounds__(RUN ? 64 * (kRunHelpers + 1) : 64) void rms_reg_ker
             f.bad[b] = static_cast<uint64_t>(lo) | (static_cast<uint64_t>(hi) << 32);
         }
         f.e0 = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(scans_lds->e0));
-        float run[kRunS];
+        float run[4];
         read_run(run);
-        sb[0] = fold_walk<kRunS, 4>(f, run, __float_as_uint(head));
+        sb[0] = fold_walk<4, 4>(f, run, __float_as_uint(head));
     }
     if (MODE == kNormAddNorm) {  // stored residual stream r = x + residual
 #pragma unroll
@@ -599,8 +590,8 @@ __global__ __launch_bounds__(RUN ? 64 * (kRunHelpers + 1) : 64) void rms_reg_ker
     // lane r's s).  A single row with the wave-parallel fold computes it
     // uniformly instead, without the readlane.  Measured on MI355X: the
     // residual epilogue at [4096, 1536] (two rows) 13.61-13.62 against
-    // 13.67-13.79 us with a chain per row; C5 at 256 rows (one) 4.74-4.79
-    // against 4.70-4.73 with the readlane.
+    // 13.67-13.79 us with a chain per row; [1, 512] (one) 2.59 against 2.67
+    // with the readlane, [700, 512] 3.94 against 4.06.
     constexpr bool kUniform = (PAR || kTail) && R == 1;
     float sum_r = s;
     if constexpr (PAR || kTail) {
