@@ -138,7 +138,7 @@ __global__ __launch_bounds__(256) void q4_0_matvec_kernel(MatvecArgs a) {
     const uint32_t tid = threadIdx.x, lane = tid % kWave;
     const uint32_t wave = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(tid / kWave));
     const uint32_t n = a.input_width, n4 = n / 4, nb = n / 32, row_bytes = nb * kQ4Block;
-    const uint32_t groups = a.groups;
+    const uint32_t groups = STAGED ? a.groups : 1u;
     const uint32_t rows = kPassRows * groups * kWaves / KS;  // rows per workgroup
 
     // The projection this workgroup's rows belong to (segments are tile ranges).
