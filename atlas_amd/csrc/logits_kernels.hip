@@ -57,14 +57,14 @@ SoftCap soft_cap(float cap) { return {cap, cap >= 0x1p-20f && cap <= 0x1p20f ? 1
 // wavefront needs it (a wave-uniform branch), then selected per value.  Bound
 // by this arithmetic where logits reach the exponential (|v| >= 0.625 cap), so
 // both divisions are shorter ones where that is exact:
-//  * v / cap in wavefronts whose |v| all lie in [2^-70, 2^60] -- ordinary
-//    logits; an exact zero, a mask's -inf or lowest float sends the wavefront
-//    to the IEEE division: q0 = v rcp is within 1.5 ulp of the quotient; q1 =
+//  * v / cap in wavefronts whose |q0| = |v rcp| all lie in [2^-70, 2^60] --
+//    ordinary logits; an exact zero, a mask's -inf or lowest float sends the
+//    wavefront to the IEEE division: q0 is within 1.5 ulp of the quotient; q1 =
 //    fma(v - q0 cap, rcp, q0) within half an ulp and a few 2^-22 of one, so
-//    faithful; and q2 = fma(v - q1 cap, rcp, q1), with the residual exact (no
-//    operand or product comes near the subnormals) and rcp correctly rounded,
-//    is the correctly rounded quotient (Markstein 1990).  Five operations
-//    against the division's eleven;
+//    faithful; and q2 = fma(v - q1 cap, rcp, q1), with the residual exact (a
+//    multiple of 2^-136; no operand comes near the subnormals) and rcp correctly
+//    rounded, is the correctly rounded quotient (Markstein 1990).  Five
+//    operations against the division's eleven;
 //  * 2 / (e^{2a} + 1): tanh_exp_abs_with, enumerated equal over its whole
 //    domain, for every wavefront.
 // With wave_key below, soft cap + argmax of [256, 262144] at logits of standard
@@ -75,20 +75,24 @@ SoftCap soft_cap(float cap) { return {cap, cap >= 0x1p-20f && cap <= 0x1p20f ? 1
 // reaches the exponential, 93 both ways.
 template <int N>
 __device__ __forceinline__ void softcap_lanes(float (&v)[N], const SoftCap& k) {
-    float hi = __builtin_fabsf(v[0]), lo = hi;
+    // the largest and smallest |q0|, not |v|: a product is never a signalling
+    // NaN, which would take what max and min hold along with it
+    float q0[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) q0[i] = v[i] * k.rcp;
+    float hi = __builtin_fabsf(q0[0]), lo = hi;
 #pragma unroll
     for (int i = 1; i < N; ++i) {
-        hi = fmaxf(hi, __builtin_fabsf(v[i]));
-        lo = fminf(lo, __builtin_fabsf(v[i]));
+        hi = fmaxf(hi, __builtin_fabsf(q0[i]));
+        lo = fminf(lo, __builtin_fabsf(q0[i]));
     }
     float a[N], r[N];
     // NaN among plain values: max and min skip it, every step propagates it
     // and the range test below leaves it to the series
-    if (k.rcp != 0.0f && __builtin_amdgcn_ballot_w64(!(hi <= 0x1p60f && lo >= 0x1p-70f)) == 0) {
+    if (__builtin_amdgcn_ballot_w64(!(hi <= 0x1p60f && lo >= 0x1p-70f)) == 0) {
 #pragma unroll
         for (int i = 0; i < N; ++i) {
-            const float q0 = v[i] * k.rcp;
-            const float q1 = __builtin_fmaf(__builtin_fmaf(-q0, k.cap, v[i]), k.rcp, q0);
+            const float q1 = __builtin_fmaf(__builtin_fmaf(-q0[i], k.cap, v[i]), k.rcp, q0[i]);
             a[i] = __builtin_fabsf(__builtin_fmaf(__builtin_fmaf(-q1, k.cap, v[i]), k.rcp, q1));
         }
     } else {
@@ -97,8 +101,8 @@ __device__ __forceinline__ void softcap_lanes(float (&v)[N], const SoftCap& k) {
     }
 #pragma unroll
     for (int i = 0; i < N; ++i) r[i] = tanh_series_abs(a[i]);
-    // the quotient rounds monotonically: below 0.6249 cap none reaches 0.625
-    if (__builtin_amdgcn_ballot_w64(hi >= 0.6249f * k.cap) != 0) {
+    // q0 is within 1.5 ulp of the quotient: below 0.6249 none reaches 0.625
+    if (__builtin_amdgcn_ballot_w64(hi >= 0.6249f || k.rcp == 0.0f) != 0) {
 #pragma unroll
         for (int i = 0; i < N; ++i) {
             const float big = tanh_exp_abs_with<DivPositive>(a[i]);
@@ -111,15 +115,24 @@ __device__ __forceinline__ void softcap_lanes(float (&v)[N], const SoftCap& k) {
 }
 
 // The wavefront's key over N float4 a lane, float4 u of lane l holding the
-// values from index first + (u * kLogitThreads + l) * 4 on: the wavefront's
-// maximum (NaN never raises it), then the last position that equals it, on the
-// scalar unit from the comparisons' lane masks -- two VALU operations a value
-// where folding a 64-bit key per value takes ten.  Wave-uniform.
-template <int N>
-__device__ __forceinline__ uint64_t wave_key(const float (&x)[4 * N], uint32_t first) {
+// values from index first + (u * kLogitThreads + l) * 4 on, or from `top` where
+// that is less: the wavefront's maximum (NaN never raises it), then the last
+// position that equals it, on the scalar unit from the comparisons' lane masks --
+// two VALU operations a value where folding a 64-bit key per value takes ten.
+// Wave-uniform.  RAW: values as loaded, which may be signalling NaNs; fmaxf loses
+// what it holds beside one, so the first maximum is the propagating one, and
+// where it is NaN a second takes the values quieted (quieting all of them:
+// [128, 151936] 16.2 -> 16.8 us).
+template <int N, bool RAW>
+__device__ __forceinline__ uint64_t wave_key(const float (&x)[4 * N], uint32_t first, uint32_t top) {
     float m = x[0];
 #pragma unroll
-    for (int i = 1; i < 4 * N; ++i) m = fmaxf(m, x[i]);
+    for (int i = 1; i < 4 * N; ++i) m = RAW ? __builtin_elementwise_maximum(m, x[i]) : fmaxf(m, x[i]);
+    if (RAW && __builtin_amdgcn_ballot_w64(m != m) != 0) {
+        m = __builtin_canonicalizef(x[0]);
+#pragma unroll
+        for (int i = 1; i < 4 * N; ++i) m = fmaxf(m, __builtin_canonicalizef(x[i]));
+    }
     m = wave_max_tree_f32(m);
     uint64_t key = 0;  // every value NaN
     bool open = true;
@@ -133,7 +146,7 @@ __device__ __forceinline__ uint64_t wave_key(const float (&x)[4 * N], uint32_t f
             open = false;
             const uint32_t lane = 63u - static_cast<uint32_t>(__builtin_clzll(any));
             const uint32_t j = (hit[3] >> lane) & 1 ? 3u : ((hit[2] >> lane) & 1 ? 2u : ((hit[1] >> lane) & 1 ? 1u : 0u));
-            key = argmax_key(m, first + (u * kLogitThreads + lane) * 4 + j);
+            key = argmax_key(m, min(first + (u * kLogitThreads + lane) * 4, top) + j);
         }
     }
     return key;
@@ -179,8 +192,10 @@ __global__ __launch_bounds__(kLogitThreads) void argmax_finish_kernel(const uint
 // multiple of 4 shifts every row); every load of a step is issued before its
 // first value is processed.  A float4 that runs past the row is loaded from
 // the row's last 4 values; the ones in front of its own position belong to
-// the thread before it and are neither stored nor counted.  [256, 50257] (one
-// value a thread before): 39.3 -> 24.8 us, argmax of [256, 32001] 16.5 -> 9.4.
+// the thread before it.  They are not stored, and the soft cap does not count
+// them (in place, that thread may have stored already); the argmax alone counts
+// them a second time, at their index.  [256, 50257] (one value a thread before):
+// 39.3 -> 24.8 us, argmax of [256, 32001] 16.5 -> 9.4.
 typedef f32x4 f32x4_row __attribute__((aligned(4)));
 
 template <bool CAP, bool ARG, int U>
@@ -224,7 +239,7 @@ __global__ __launch_bounds__(kLogitThreads) void logits_vec_kernel(const float* 
                         if (count - 4 + j >= i) out[base + count - 4 + j] = x[4 * u + j];
                 }
             }
-            if (ARG && !whole) {
+            if (CAP && ARG && !whole) {
                 // position j of this float4 is index i + j: shift the tail's
                 // values down and fill with NaN, which never wins
                 const uint32_t skip = i + 4 <= last ? 0u : (i < last ? i + 4 - last : 4u);
@@ -240,7 +255,7 @@ __global__ __launch_bounds__(kLogitThreads) void logits_vec_kernel(const float* 
                 for (int j = 0; j < 4; ++j) x[4 * u + j] = y[j];
             }
         }
-        if (ARG) key = max_u64(key, wave_key<U>(x, begin + wave * (kWave * 4)));
+        if (ARG) key = max_u64(key, wave_key<U, !CAP>(x, begin + wave * (kWave * 4), CAP ? 0xffffffffu : count - 4));
     }
     if (ARG) publish_key<true>(key, row, slots, selected);
 }

@@ -108,6 +108,32 @@ def test_special_values(rt, ora, rows, count, std):
         rt.free(b)
 
 
+# a signalling NaN is a value like any other NaN: what its lane holds before it
+# still counts, for the argmax and for the choice of the soft cap's steps (one
+# float4 a lane, and four, 1024 values apart)
+@pytest.mark.parametrize("rows,count,apart", [(2, 3000, (1, 2, 3)), (1100, 4096, (1, 3, 1024, 2049, 3074))])
+@pytest.mark.parametrize("first", [25.0, 1e30, np.inf, 1e-45])
+def test_signalling_nan(rt, ora, rows, count, apart, first):
+    r = np.random.default_rng(count)
+    x = r.standard_normal((rows, count)).astype(f32)
+    for i in range(rows):
+        at = 4 * (i % 250)
+        x[i, at] = first
+        x[i].view(np.uint32)[at + apart[i % len(apart)]] = 0x7F800001 if i % 2 else 0xFFBFFFFF
+    x = x.reshape(-1)
+    exp_c, exp_s = ora.softcap_argmax_rows(x, rows, count, 30.0)
+    src, dst, sel = rt.upload(x), rt.empty(x.size), rt.empty(rows, np.uint32)
+    rt.softcap_argmax(src, dst, sel, rows, count, 30.0)
+    rt.sync()
+    assert _same(dst.download(x.size), exp_c)
+    assert np.array_equal(sel.download(rows, np.uint32), exp_s)
+    rt.argmax(src, sel, rows, count)
+    rt.sync()
+    assert np.array_equal(sel.download(rows, np.uint32), ora.softcap_argmax_rows(x, rows, count, 0.0)[1])
+    for b in (src, dst, sel):
+        rt.free(b)
+
+
 def test_in_range_division_is_ieee_on_the_exponential_range():
     # every float from 0.625 to infinity, as test_gpu_division does for the activations
     counts = (ctypes.c_uint64 * 4)()
