@@ -447,8 +447,8 @@ hipError_t launch_exact_mode(hipStream_t s, const NormArgs& a) {
     return launch_exact<4, 8, 1, 2, MODE>(s, a);
 }
 
-// [1000, 4096] plain 8.2 us (16.0 with one wavefront per row reading it
-// twice), [4096, 4096] 24.3 (37.7); one row 2.5 (5.8).
+// [1000, 4096] plain 7.4 us (16.3 with one wavefront per row reading it
+// twice), [4096, 4096] 24.0 (36.9); one row 2.5 (5.8).
 template <int MODE>
 hipError_t launch_tree_mode(hipStream_t s, const NormArgs& a) {
     const uint32_t h = a.hidden;

@@ -1,6 +1,6 @@
-"""The Q4_0 projections' integer dot: every launch form (a quarter of a row per
-wavefront, a row's blocks loaded by their lanes, staged rows in one, two and
-four groups) at its edges, against the float64 oracle, and inputs whose digits
+"""The Q4_0 projections' integer dot: every launch form (a quarter and a half of a
+row per wavefront, a row's blocks loaded by their lanes, staged rows in one, two
+and four groups) at its edges, against the float64 oracle, and inputs whose digits
 need care: mixed magnitudes inside a block, subnormals, the largest floats,
 infinities and NaN."""
 import matvec_cases as mc
